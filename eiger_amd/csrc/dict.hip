@@ -398,8 +398,10 @@ DevBuf dict_encode(const void* keys, int64_t n, const void* dict, int64_t m, int
     if (n == 0) return out;
     if (m > kMaxDict) raise(EG_ERR_UNSUPPORTED, "dictionary larger than 2^30 entries");
     if (m > 0) {
-        uint64_t tmin = 0, tmax = 0;
-        key_range(dict, type, kb, m, s, &tmin, &tmax);  // order-preserving form
+        KeyRange range;  // order-preserving form
+        const RangeCol rc{dict, type, kb};
+        key_ranges(&rc, 1, m, s, &range);
+        const uint64_t tmin = range.min, tmax = range.max;
         const uint64_t span = tmax - tmin;
         if (span < (uint64_t)kDirectMax) {
             const uint64_t raw_min = twiddle_bits(tmin, type, kb);  // the twiddle of an integer is its own inverse

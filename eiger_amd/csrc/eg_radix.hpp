@@ -74,7 +74,17 @@ __host__ __device__ inline uint64_t twiddle_bits(uint64_t raw, int32_t type, int
     return raw;
 }
 
-// Min and max of the twiddled keys (device reduction, synchronises s).
-void key_range(const void* keys, int32_t type, int bytes, int64_t n, hipStream_t s, uint64_t* mn, uint64_t* mx);
+// Range of the twiddled keys of each column (n rows each): minimum, maximum
+// and the bits that are not the same in every key.  One synchronisation of s
+// per 16 columns.
+struct RangeCol {
+    const void* data;
+    int32_t type;
+    int32_t bytes;
+};
+struct KeyRange {
+    uint64_t min, max, varying;
+};
+void key_ranges(const RangeCol* cols, int ncols, int64_t n, hipStream_t s, KeyRange* out);
 
 }  // namespace eg

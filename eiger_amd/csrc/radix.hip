@@ -395,33 +395,58 @@ void scan_rec(const uint32_t* in, uint32_t* out, int64_t n, hipStream_t s)
 }
 
 // ---- key range ----------------------------------------------------------------------
-__global__ __launch_bounds__(256) void key_range_kernel(const void* keys, int32_t type, int bytes, int64_t n,
-                                                        unsigned long long* mn, unsigned long long* mx)
+// Every block leaves its minimum, maximum, OR and AND of the radix-ordered
+// keys; the host folds the blocks' words (at most 512 x 4, one copy).  No
+// atomics: with a pair of same-address atomics per wave their serialisation
+// (~80 per microsecond) was the whole kernel -- 40M int64 keys 239 us, now
+// the read of the keys.
+constexpr int kRangeB = 512;
+constexpr int kRangeGrid = 512;  // two blocks of eight waves per CU
+
+template <int KB>
+__global__ __launch_bounds__(kRangeB) void key_range_kernel(const void* __restrict__ keys, int32_t type, int64_t n,
+                                                            unsigned long long* __restrict__ out)
 {
-    uint64_t lo = ~0ull, hi = 0ull;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const uint64_t v = twiddle_bits(dev::load_raw(keys, bytes, i), type, bytes);
+    __shared__ unsigned long long sh[kRangeB / 64][4];
+    uint64_t lo = ~0ull, hi = 0ull, any = 0ull, all = ~0ull;
+    auto take = [&](uint64_t raw) {
+        const uint64_t v = twiddle_bits(raw, type, KB);
         lo = v < lo ? v : lo;
         hi = v > hi ? v : hi;
+        any |= v;
+        all &= v;
+    };
+    const int64_t stride = (int64_t)gridDim.x * kRangeB;
+    int64_t i = (int64_t)blockIdx.x * kRangeB + threadIdx.x;
+    for (; i + 7 * stride < n; i += 8 * stride) {  // eight loads in flight
+        uint64_t raw[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) raw[j] = load_key<KB>(keys, i + j * stride);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) take(raw[j]);
     }
+    for (; i < n; i += stride) take(load_key<KB>(keys, i));
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
         const uint64_t a = __shfl_xor((unsigned long long)lo, off), b = __shfl_xor((unsigned long long)hi, off);
         lo = a < lo ? a : lo;
         hi = b > hi ? b : hi;
+        any |= __shfl_xor((unsigned long long)any, off);
+        all &= __shfl_xor((unsigned long long)all, off);
     }
     if ((threadIdx.x & 63) == 0) {
-        atomicMin(mn, (unsigned long long)lo);
-        atomicMax(mx, (unsigned long long)hi);
+        unsigned long long* w = sh[threadIdx.x >> 6];
+        w[0] = lo, w[1] = hi, w[2] = any, w[3] = all;
     }
-}
-
-__global__ void init_range_kernel(unsigned long long* p)
-{
-    if (threadIdx.x == 0) {
-        p[0] = ~0ull;
-        p[1] = 0ull;
+    __syncthreads();
+    if (threadIdx.x < 4) {
+        const int q = threadIdx.x;
+        unsigned long long r = sh[0][q];
+        for (int w = 1; w < kRangeB / 64; ++w) {
+            const unsigned long long x = sh[w][q];
+            r = q == 0 ? (x < r ? x : r) : q == 1 ? (x > r ? x : r) : q == 2 ? (r | x) : (r & x);
+        }
+        out[(int64_t)blockIdx.x * 4 + q] = r;
     }
 }
 
@@ -442,23 +467,42 @@ uint64_t scan_exclusive_u32(const uint32_t* in, uint32_t* out, int64_t n, hipStr
     return (uint64_t)h[0];
 }
 
-void key_range(const void* keys, int32_t type, int bytes, int64_t n, hipStream_t s, uint64_t* mn, uint64_t* mx)
+void key_ranges(const RangeCol* cols, int ncols, int64_t n, hipStream_t s, KeyRange* out)
 {
-    DevBuf r(16, s);
-    hipLaunchKernelGGL(init_range_kernel, dim3(1), dim3(64), 0, s, r.get<unsigned long long>());
-    EG_LAUNCH_CHECK();
-    if (n > 0) {
-        const int64_t grid = std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, (int64_t)device_info().num_cus * 8));
-        KernelTimer timer("key_range", s);
-        hipLaunchKernelGGL(key_range_kernel, dim3((unsigned)grid), dim3(256), 0, s, keys, type, bytes, n,
-                           r.get<unsigned long long>(), r.get<unsigned long long>() + 1);
-        EG_LAUNCH_CHECK();
+    for (int c = 0; c < ncols; ++c) out[c] = KeyRange{~0ull, 0ull, 0ull};
+    if (n <= 0) return;
+    const int64_t grid = std::max<int64_t>(1, std::min<int64_t>((n + kRangeB * 8 - 1) / (kRangeB * 8), kRangeGrid));
+    constexpr int kGroup = 16;  // columns per synchronisation
+    for (int c0 = 0; c0 < ncols; c0 += kGroup) {
+        const int m = std::min(kGroup, ncols - c0);
+        const size_t words = (size_t)grid * 4;
+        DevBuf part((size_t)m * words * 8, s);
+        unsigned long long* p = part.get<unsigned long long>();
+        for (int c = 0; c < m; ++c) {
+            const RangeCol& col = cols[c0 + c];
+            KernelTimer timer("key_range", s);
+            auto kern = col.bytes == 1 ? key_range_kernel<1> : col.bytes == 2 ? key_range_kernel<2>
+                      : col.bytes == 4 ? key_range_kernel<4> : key_range_kernel<8>;
+            hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kRangeB), 0, s, col.data, col.type, n, p + c * words);
+            EG_LAUNCH_CHECK();
+        }
+        const uint64_t* h = (const uint64_t*)pinned_staging((size_t)m * words * 8, 3);
+        EG_HIP(hipMemcpyAsync((void*)h, p, (size_t)m * words * 8, hipMemcpyDeviceToHost, s));
+        EG_HIP(hipStreamSynchronize(s));
+        for (int c = 0; c < m; ++c) {
+            KeyRange r{~0ull, 0ull, 0ull};
+            uint64_t any = 0ull, all = ~0ull;
+            for (int64_t b = 0; b < grid; ++b) {
+                const uint64_t* w = h + (size_t)c * words + (size_t)b * 4;
+                r.min = std::min(r.min, w[0]);
+                r.max = std::max(r.max, w[1]);
+                any |= w[2];
+                all &= w[3];
+            }
+            r.varying = any & ~all;
+            out[c0 + c] = r;
+        }
     }
-    int64_t* h = pinned_i64(2);
-    EG_HIP(hipMemcpyAsync(h, r.get(), 16, hipMemcpyDeviceToHost, s));
-    EG_HIP(hipStreamSynchronize(s));
-    *mn = (uint64_t)h[0];
-    *mx = (uint64_t)h[1];
 }
 
 void radix_pass(const RadixKeys& k, void* keys_out, const std::vector<Payload>& pay, int64_t n, int shift,

@@ -235,10 +235,14 @@ void fuse_keys(const ViewIn* keys, int64_t ncols, hipStream_t s, FusedKeys& f)
         }
         f.type[c] = t;
         f.bytes[c] = type_size(t);
-        uint64_t mn = 0, mx = 0;
-        if (n > 0) key_range(src[c], t, f.bytes[c], n, s, &mn, &mx);
-        f.min[c] = mn;
-        f.bits[c] = bit_width(mx - mn);
+    }
+    std::vector<RangeCol> rcol((size_t)ncols);
+    std::vector<KeyRange> range((size_t)ncols, KeyRange{0, 0, 0});
+    for (int64_t c = 0; c < ncols; ++c) rcol[c] = RangeCol{src[c], f.type[c], f.bytes[c]};
+    if (n > 0) key_ranges(rcol.data(), (int)ncols, n, s, range.data());
+    for (int64_t c = 0; c < ncols; ++c) {
+        f.min[c] = range[c].min;
+        f.bits[c] = bit_width(range[c].max - range[c].min);
         total += f.bits[c];
     }
     if ((total > 64 || ncols > kMaxFuseItems) && n >= ((int64_t)1 << 32))
