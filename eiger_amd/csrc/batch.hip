@@ -46,6 +46,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "eg_atomics.hpp"
@@ -80,8 +81,10 @@ struct BQuery {
     int64_t scratch_off;  // its rows in the partitioned scratch columns
 };
 
-// A work item: rows [begin, end) of query q (kind 0), or partition `begin`
-// of a partitioned query (kind 1).
+// A work item: rows [begin, end) of query q, one of several such items
+// (merged through its HBM table) or all of its rows (groups straight to the
+// output), or partition `begin` of a partitioned query.
+enum : int32_t { kItemRows = 0, kItemPart = 1, kItemWhole = 2 };
 struct BItem {
     int32_t q;
     int32_t kind;
@@ -127,7 +130,7 @@ __device__ __forceinline__ GTable query_table(const BQuery& q, int W, unsigned l
     return gt;
 }
 
-// meta words per query: [0] inserts (unused), [1] side slot used, [2] full
+// meta words per query: [0] HBM-table inserts, [1] side slot used, [2] full
 constexpr int kMetaWords = 4;
 
 __global__ void batch_fill_kernel(unsigned long long* p, uint64_t words)
@@ -167,24 +170,37 @@ __global__ __launch_bounds__(kPB) void bpart_hist_kernel(const BQuery* __restric
 
 // Exclusive scan of one partitioned query's counts in [partition][tile]
 // order (in place): each entry becomes the query-local row where that tile's
-// rows of that partition start.  One 1024-thread workgroup per query, 8
-// entries per thread per round.
+// rows of that partition start.  One 1024-thread workgroup per query; every
+// wave sums its sixteenth of the counts, then scans it from the sum of the
+// waves before, so only two barriers are serial (walking the counts in
+// workgroup-wide rounds took 228 us on the largest query of 512, 250k counts).
 __global__ __launch_bounds__(1024) void bpart_scan_kernel(const BQuery* __restrict__ qs, const int32_t* __restrict__ pqs,
                                                           uint32_t* __restrict__ hist)
 {
-    constexpr int K = 8;
+    constexpr int K = 4;  // counts per lane per step
     __shared__ uint32_t wsum[16];
     const BQuery& q = qs[pqs[blockIdx.x]];
     const int64_t n = ((int64_t)1 << q.pbits) * q.ntiles;
     uint32_t* a = hist + q.hist_off;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t per = (n + 16 * 64 * K - 1) / (16 * 64 * K) * (64 * K);  // counts per wave
+    const int64_t b = w * per, e = min(n, b + per);
+    uint32_t sum = 0;
+#pragma unroll 4
+    for (int64_t i = b + lane; i < e; i += 64) sum += a[i];
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off);
+    if (lane == 0) wsum[w] = sum;
+    __syncthreads();
     uint32_t carry = 0;
-    for (int64_t base = 0; base < n; base += (int64_t)K * blockDim.x) {
-        const int64_t i0 = base + (int64_t)threadIdx.x * K;
+    for (int i = 0; i < w; ++i) carry += wsum[i];
+#pragma unroll 2
+    for (int64_t base = b; base < e; base += 64 * K) {
+        const int64_t i0 = base + lane * K;
         uint32_t v[K], tot = 0;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            v[k] = i0 + k < n ? a[i0 + k] : 0u;
+            v[k] = i0 + k < e ? a[i0 + k] : 0u;
             tot += v[k];
         }
         uint32_t x = tot;  // inclusive scan over the wave
@@ -193,21 +209,13 @@ __global__ __launch_bounds__(1024) void bpart_scan_kernel(const BQuery* __restri
             const uint32_t y = __shfl_up(x, off);
             if (lane >= off) x += y;
         }
-        if (lane == 63) wsum[w] = x;
-        __syncthreads();
-        uint32_t before = carry, round = 0;
-        for (int i = 0; i < 16; ++i) {
-            if (i < w) before += wsum[i];
-            round += wsum[i];
-        }
-        uint32_t ex = before + x - tot;
+        uint32_t ex = carry + x - tot;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            if (i0 + k < n) a[i0 + k] = ex;
+            if (i0 + k < e) a[i0 + k] = ex;
             ex += v[k];
         }
-        carry += round;
-        __syncthreads();  // wsum is reused
+        carry += __shfl(x, 63);
     }
 }
 
@@ -270,26 +278,164 @@ __device__ __forceinline__ void emit_batch(const BOut& bo, const BQuery& q, int6
     }
 }
 
+// The requests' ops (at most EG_BATCH_MAX_AGGS) in one word: an OpCode byte
+// each, 0xff past the last.  A scalar branch on the byte reaches code with the
+// operand transform and the atomic compiled in; the ops as kernel-argument
+// structs took 180 scalar registers more than there are.
+struct BOps {
+    uint32_t codes;
+    int32_t conv;     // value conversion (ConvCode)
+    int32_t has_any;  // an exchange among them: no partial states in registers
+
+    template <class F>
+    __device__ __forceinline__ void each(F&& f) const
+    {
+#pragma unroll
+        for (int a = 0; a < EG_BATCH_MAX_AGGS; ++a) {
+            switch ((codes >> (8 * a)) & 0xffu) {  // uniform
+            case OPC_COUNT: f(a, std::integral_constant<int, OPC_COUNT>{}); break;
+            case OPC_SUM_I:
+            case OPC_SUM_U: f(a, std::integral_constant<int, OPC_SUM_U>{}); break;
+            case OPC_SUM_F: f(a, std::integral_constant<int, OPC_SUM_F>{}); break;
+            case OPC_MAX_I: f(a, std::integral_constant<int, OPC_MAX_I>{}); break;
+            case OPC_MAX_U: f(a, std::integral_constant<int, OPC_MAX_U>{}); break;
+            case OPC_MAX_F: f(a, std::integral_constant<int, OPC_MAX_F>{}); break;
+            case OPC_MIN_I: f(a, std::integral_constant<int, OPC_MIN_I>{}); break;
+            case OPC_MIN_U: f(a, std::integral_constant<int, OPC_MIN_U>{}); break;
+            case OPC_MIN_F: f(a, std::integral_constant<int, OPC_MIN_F>{}); break;
+            case OPC_ANY: f(a, std::integral_constant<int, OPC_ANY>{}); break;
+            default: break;
+            }
+        }
+    }
+    template <int CODE>
+    __device__ __forceinline__ static uint64_t operand(uint64_t v)
+    {
+        if constexpr (CODE == OPC_COUNT) return 1ull;
+        else return v ^ op_xmask(CODE) ^ ((uint64_t)((int64_t)v >> 63) & op_fmask(CODE));
+    }
+};
+
+// A plan's constants in device memory.
+struct BConst {
+    AggSpec spec;
+    BOut bo;
+};
+
+// One value of VB bytes (0: no value column; -1: any width, read at run time).
+template <int VB>
+__device__ __forceinline__ uint64_t load_value(const void* p, int vbytes, int64_t r)
+{
+    if constexpr (VB == 0) return 0ull;
+    else if constexpr (VB == 4) return ((const uint32_t*)p)[r];
+    else if constexpr (VB == 8) return ((const uint64_t*)p)[r];
+    else return dev::load_raw(p, vbytes, r);
+}
+
+// Fewest of a step's first rows holding lane 0's key for a wave to keep that
+// key's partial states in registers (see hash_agg's rule).
+constexpr int kBatchHot = 8;
+
+// Rows [b, e) of (keys, vals) into the workgroup's LDS table, spilling to gt.
+// Four rows a lane per step, their loads issued together; each lane probes
+// and updates for itself.  A key that many lanes hold accumulates in
+// registers and reaches its slot with one wave reduction.  Walking one row a
+// lane with wave-level combining for every row took 3.9 ms for the 512-query
+// mix (247M rows) instead of this loop's time.
+template <int KB, int VB>
+__device__ __forceinline__ void batch_rows(LdsTable<KB, true>& tab, const GTable& gt, const KeyDesc& key, const BOps& ops,
+                                           const void* keys, const void* vals, int vbytes, int64_t b0, int64_t e,
+                                           int probe_limit, uint32_t& ins)
+{
+    constexpr int J = 4;
+    using KT = typename LdsKey<KB>::T;
+    const int lane = dev::lane_id();
+    auto key_at = [&](int64_t r) -> uint64_t {
+        return KB == 4 ? (uint64_t)((const uint32_t*)keys)[r] : ((const uint64_t*)keys)[r];
+    };
+    auto enc = [&](uint64_t raw) -> KT {
+        return KB == 4 ? (KT)((uint32_t)raw ^ dev::kSign32) : (KT)dev::enc64(dev::widen_key(raw, KB, key.is_signed));
+    };
+    // val(a, code): the value merged into state a
+    auto add = [&](uint64_t raw, auto val) {
+        const int slot = tab.find(enc(raw), 0, probe_limit);
+        if (slot >= 0) {
+            ops.each([&](int a, auto c) { dev::apply_atomic(op_class(c), &tab.st[(size_t)a * tab.T + slot], val(a, c)); });
+        } else {  // the table is full: a cold key spills
+            unsigned long long* g = gt_slot(gt, dev::enc64(dev::widen_key(raw, KB, key.is_signed)), ins);
+            if (g) ops.each([&](int a, auto c) { dev::apply_atomic(op_class(c), g + 1 + a, val(a, c)); });
+        }
+    };
+    uint64_t acc[EG_BATCH_MAX_AGGS], hot_key = ~0ull;  // wave-uniform key
+    bool on = false;                                   // wave-uniform: acc holds rows of hot_key
+    auto flush = [&]() {
+        if (!on) return;
+        ops.each([&](int a, auto c) { acc[a] = dev::wave_reduce(op_class(c), acc[a]); });
+        if (lane == 0) add(hot_key, [&](int a, auto) { return acc[a]; });
+#pragma unroll
+        for (int a = 0; a < EG_BATCH_MAX_AGGS; ++a) acc[a] = 0ull;
+        on = false;
+    };
+#pragma unroll
+    for (int a = 0; a < EG_BATCH_MAX_AGGS; ++a) acc[a] = 0ull;
+    const int64_t step = (int64_t)J * blockDim.x;
+    for (int64_t b = b0; b < e; b += step) {
+        uint64_t kr[J], vr[J];
+        bool valid[J];
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            const int64_t r = b + (int64_t)j * blockDim.x + threadIdx.x;
+            valid[j] = r < e;
+            const int64_t src = valid[j] ? r : b0;  // in bounds, masked below
+            kr[j] = key_at(src);
+            vr[j] = load_value<VB>(vals, vbytes, src);
+        }
+        if (!ops.has_any) {
+            const uint64_t k0 = dev::readlane64(kr[0], 0);  // lane 0's key; a row of this wave's or row b0
+            if (!(on && k0 == hot_key)) {
+                const int c0 = __popcll(__ballot(valid[0] && kr[0] == k0));
+                const int ch = on ? __popcll(__ballot(valid[0] && kr[0] == hot_key)) : 0;
+                if (c0 >= kBatchHot && c0 > 2 * ch) {
+                    flush();
+                    hot_key = k0;
+                    on = true;
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            if (!valid[j]) continue;
+            const uint64_t v = dev::canon(vr[j], ops.conv);
+            if (on && kr[j] == hot_key) {
+                ops.each([&](int a, auto c) {
+                    acc[a] = dev::combine(op_class(c), acc[a], BOps::operand<decltype(c)::value>(v));
+                });
+            } else {
+                add(kr[j], [&](int, auto c) { return BOps::operand<decltype(c)::value>(v); });
+            }
+        }
+    }
+    flush();
+}
+
 // Eight waves per SIMD, so two workgroups fit a CU (blocks_per_cu = 2).
-template <int KB, int NV>
+template <int KB, int VB>
 __global__ __launch_bounds__(kBatchBlock, 8) void batch_agg_kernel(const BQuery* __restrict__ qs,
                                                                 const BItem* __restrict__ items, int n_items,
                                                                 unsigned int* next_item, unsigned long long* metas,
-                                                                AggSpec spec, int key_signed, int vbytes, int W,
-                                                                int cr_log2, int probe_limit, int peel_min,
-                                                                const uint32_t* __restrict__ offs, const void* skeys,
-                                                                const void* svals, unsigned long long* counts,
-                                                                uint32_t* qstatus, BOut bo)
+                                                                const BConst* bc, BOps ops, int nops, int key_signed,
+                                                                int vbytes, int W, int cr_log2, int probe_limit,
+                                                                int peel_min, const uint32_t* __restrict__ offs,
+                                                                const void* skeys, const void* svals,
+                                                                unsigned long long* counts, uint32_t* qstatus)
 {
     extern __shared__ __align__(16) unsigned long long smem[];
     __shared__ int s_item;
     __shared__ unsigned long long sh[17];
-    const int nops = spec.nops;
     const int lane = dev::lane_id();
     LdsTable<KB, true> tab(smem, nops, 1 << cr_log2, 0);
     const int words = LdsTable<KB>::words(nops, 1 << cr_log2, 0);
-    uint32_t ins = 0;
-    dev::HotTags hot;  // groups the wave combined last
+    dev::HotTags hot;  // groups the wave combined last (no LDS stage)
     KeyDesc key;
     key.bytes = KB;
     key.is_signed = key_signed;
@@ -300,38 +446,68 @@ __global__ __launch_bounds__(kBatchBlock, 8) void batch_agg_kernel(const BQuery*
         if (it >= n_items) break;  // the same value in every thread: the whole block leaves
         const BItem w = items[it];
         const BQuery q = qs[w.q];
-        const GTable gt = query_table(q, W, metas + (size_t)w.q * kMetaWords);
-        if (w.kind == 1) {
-            // One partition of a partitioned query: its rows from the scratch
-            // columns into the LDS table, its groups straight to the output.
+        unsigned long long* meta = metas + (size_t)w.q * kMetaWords;
+        const GTable gt = query_table(q, W, meta);
+        uint32_t ins = 0;  // HBM-table insertions by this lane
+        // the plan's constants are read where they are used (opaque pointer:
+        // not kept in scalar registers across the row loop)
+        const BConst* con = bc;
+        asm volatile("" : "+s"(con));
+        const AggSpec& spec = con->spec;
+        const BOut& bo = con->bo;
+        if (w.kind == kItemRows && q.use_lds == 0) {
+            // no LDS stage: wave-combined atomics on the HBM table
+            constexpr int NV = 1;
+            key.data = q.keys;
+            for (int64_t b = w.begin; b < w.end; b += blockDim.x) {
+                const int64_t r = b + threadIdx.x;
+                const bool valid = r < w.end;
+                const uint64_t kraw = valid ? dev::load_raw(q.keys, KB, r) : 0ull;
+                uint64_t cv[NV];
+                cv[0] = valid ? dev::canon(load_value<VB>(q.vals, vbytes, r), ops.conv) : 0ull;
+                if (__ballot(valid) != 0ull) hbm_rows<dev::RtOps, KB, NV>(gt, key, spec, valid, kraw, cv, peel_min, ins, hot);
+            }
+            gt_count_inserts(gt, ins);
+            __syncthreads();  // s_item is reused by the next item
+            continue;
+        }
+        const void* rk = q.keys;
+        const void* rv = q.vals;
+        int64_t rb = w.begin, re = w.end;
+        if (w.kind == kItemPart) {
+            // a partition of a partitioned query: its rows in the scratch columns
             const uint32_t d = (uint32_t)w.begin;
             const uint32_t* o = offs + q.hist_off;
-            const int64_t pb = q.scratch_off + (int64_t)o[(int64_t)d * q.ntiles];
-            const int64_t pe = q.scratch_off + (d + 1 < (1u << q.pbits) ? (int64_t)o[(int64_t)(d + 1) * q.ntiles] : q.rows);
-            key.data = skeys;
-            for (int i = threadIdx.x; i < words; i += blockDim.x) smem[i] = 0ull;
-            __syncthreads();
-            for (int64_t b = pb; b < pe; b += blockDim.x) {
-                const int64_t r = b + threadIdx.x;
-                const bool valid = r < pe;
-                const uint64_t kraw = valid ? dev::load_raw(skeys, KB, r) : 0ull;
-                uint64_t cv[NV];
-#pragma unroll
-                for (int c = 0; c < NV; ++c)
-                    cv[c] = (valid && spec.nvcols > 0) ? dev::canon(dev::load_raw(svals, vbytes, r), spec.cols[0].conv) : 0ull;
-                const bool sp = lds_row<dev::RtOps, KB, NV>(tab, true, 0, lane, key, spec, kraw, cv, valid, probe_limit, peel_min, hot);
-                if (__ballot(sp) != 0ull) hbm_rows<dev::RtOps, KB, NV>(gt, key, spec, sp, kraw, cv, 65, ins, hot);
+            rb = q.scratch_off + (int64_t)o[(int64_t)d * q.ntiles];
+            re = q.scratch_off + (d + 1 < (1u << q.pbits) ? (int64_t)o[(int64_t)(d + 1) * q.ntiles] : q.rows);
+            rk = skeys;
+            rv = svals;
+        }
+        for (int i = threadIdx.x; i < words; i += blockDim.x) smem[i] = 0ull;
+        __syncthreads();
+        batch_rows<KB, VB>(tab, gt, key, ops, rk, rv, vbytes, rb, re, probe_limit, ins);
+        __syncthreads();
+        using KT = typename LdsKey<KB>::T;
+        auto slot_key = [&](int sl, KT& kw) {
+            kw = 0;
+            if (sl < tab.cr) {
+                kw = tab.keys[sl];
+                return kw != 0;
             }
-            __syncthreads();
-            using KT = typename LdsKey<KB>::T;
-            auto slot_key = [&](int sl, KT& kw) {
-                kw = 0;
-                if (sl < tab.cr) {
-                    kw = tab.keys[sl];
-                    return kw != 0;
-                }
-                return sl == tab.cr && tab.side[0] != 0ull;
-            };
+            return sl == tab.cr && tab.side[0] != 0ull;
+        };
+        if (w.kind == kItemRows) {
+            // other items hold rows of this query too: merge into its HBM table
+            for (int s = threadIdx.x; s <= tab.cr; s += blockDim.x) {
+                KT kw;
+                if (!slot_key(s, kw)) continue;
+                unsigned long long* g = gt_slot(gt, lds_to_enc64<KB>(kw, key_signed), ins);
+                if (!g) continue;
+                dev::merge_states<dev::RtOps>(spec, [&](int a) { return g + 1 + a; },
+                                              [&](int a) { return tab.st[(size_t)a * tab.T + s]; });
+            }
+        } else {
+            // a partition, or a whole query: its groups straight to the output
             const int wv = threadIdx.x >> 6;
             const int nw = (blockDim.x + 63) >> 6;
             uint32_t wave_groups = 0;
@@ -364,76 +540,51 @@ __global__ __launch_bounds__(kBatchBlock, 8) void batch_agg_kernel(const BQuery*
                 }
                 pos += __popcll(m);
             }
-            __syncthreads();  // LDS, sh and s_item are reused by the next item
-            continue;
         }
-        key.data = q.keys;
-        const bool use_lds = q.use_lds != 0;
-        if (use_lds) {
-            for (int i = threadIdx.x; i < words; i += blockDim.x) smem[i] = 0ull;
-            __syncthreads();
-        }
-        for (int64_t b = w.begin; b < w.end; b += blockDim.x) {
-            const int64_t r = b + threadIdx.x;
-            const bool valid = r < w.end;
-            const uint64_t kraw = valid ? dev::load_raw(q.keys, KB, r) : 0ull;
-            uint64_t cv[NV];
-#pragma unroll
-            for (int c = 0; c < NV; ++c)
-                cv[c] = (valid && spec.nvcols > 0) ? dev::canon(dev::load_raw(q.vals, vbytes, r), spec.cols[0].conv)
-                                                   : 0ull;
-            bool sp = valid;
-            if (use_lds) sp = lds_row<dev::RtOps, KB, NV>(tab, true, 0, lane, key, spec, kraw, cv, valid, probe_limit, peel_min, hot);
-            if (__ballot(sp) != 0ull) hbm_rows<dev::RtOps, KB, NV>(gt, key, spec, sp, kraw, cv, use_lds ? 65 : peel_min, ins, hot);
-        }
-        if (use_lds) {
-            __syncthreads();
-            for (int s = threadIdx.x; s <= tab.cr; s += blockDim.x) {
-                typename LdsKey<KB>::T kw = 0;
-                if (s == tab.cr) {
-                    if (tab.side[0] == 0ull) continue;
-                } else {
-                    kw = tab.keys[s];
-                    if (kw == 0) continue;
-                }
-                unsigned long long* g = gt_slot(gt, lds_to_enc64<KB>(kw, key_signed), ins);
-                if (!g) continue;
-                dev::merge_states<dev::RtOps>(spec, [&](int a) { return g + 1 + a; },
-                                  [&](int a) { return tab.st[(size_t)a * tab.T + s]; });
-            }
-        }
-        __syncthreads();  // LDS and s_item are reused by the next item
+        gt_count_inserts(gt, ins);
+        __syncthreads();  // LDS, sh and s_item are reused by the next item
     }
 }
 
-__global__ void batch_compact_kernel(const BQuery* __restrict__ qs, const BCItem* __restrict__ citems,
-                                     unsigned long long* metas, unsigned long long* counts, uint32_t* qstatus,
-                                     BOut bo, int W)
+// A range of one query's HBM table to its outputs: kCompactSlots slots per
+// thread per round, one claim per round (a slot per thread and round left a
+// 2^16-slot range 256 rounds of three barriers: 305 us for the 512-query mix).
+__global__ __launch_bounds__(256) void batch_compact_kernel(const BQuery* __restrict__ qs,
+                                                            const BCItem* __restrict__ citems, unsigned long long* metas,
+                                                            unsigned long long* counts, uint32_t* qstatus,
+                                                            const BConst* bc, int W)
 {
+    constexpr int R = kCompactSlots;
     __shared__ unsigned long long sh[17];
     const BCItem c = citems[blockIdx.x];
-    const BQuery q = qs[c.q];
     unsigned long long* meta = metas + (size_t)c.q * kMetaWords;
     if (c.slot_begin == 0 && threadIdx.x == 0 && meta[2] != 0ull) atomicOr(&qstatus[c.q], kStTableFull);
-    for (uint64_t base = c.slot_begin; base < c.slot_end; base += blockDim.x) {
-        const uint64_t s = base + threadIdx.x;
-        bool occ = false;
-        const unsigned long long* slot = nullptr;
-        uint64_t enc = 0;
-        if (s < c.slot_end) {
+    if (meta[0] == 0ull && meta[1] == 0ull) return;  // nothing reached this query's HBM table
+    const BQuery q = qs[c.q];
+    const BOut& bo = bc->bo;
+    for (uint64_t base = c.slot_begin; base < c.slot_end; base += (uint64_t)blockDim.x * R) {
+        uint64_t enc[R];
+        uint32_t occ = 0;
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const uint64_t s = base + (uint64_t)i * blockDim.x + threadIdx.x;
+            enc[i] = 0;
+            if (s >= c.slot_end) continue;
             if (s <= q.mask) {
-                slot = q.table + s * (uint64_t)W;
-                enc = slot[0];
-                occ = enc != 0;
-            } else {
-                slot = q.table + (q.mask + 1) * (uint64_t)W;  // side slot: key 0 encoding
-                occ = meta[1] != 0;
+                enc[i] = q.table[s * (uint64_t)W];
+                if (enc[i] != 0) occ |= 1u << i;
+            } else if (meta[1] != 0) {  // the side slot: key encoding 0
+                occ |= 1u << i;
             }
         }
-        const int64_t idx = dev::block_claim(&counts[c.q], occ, sh);
-        if (occ) {
-            if (idx < q.capacity) emit_batch(bo, q, idx, enc, slot + 1, 1);
+        int64_t idx = dev::block_claim_n(&counts[c.q], (uint32_t)__popc(occ), sh);
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            if (!((occ >> i) & 1u)) continue;
+            const uint64_t s = base + (uint64_t)i * blockDim.x + threadIdx.x;
+            if (idx < q.capacity) emit_batch(bo, q, idx, enc[i], q.table + s * (uint64_t)W + 1, 1);
             else atomicOr(&qstatus[c.q], kStCapacity);
+            ++idx;
         }
     }
 }
@@ -453,9 +604,11 @@ struct BatchPlan {
     int32_t key_type = 0, val_type = 0;
     int kb = 4, vbytes = 8, nv = 0;
     AggSpec spec{};
+    BOps ops{};
     BOut bo{};
     int W = 0;
     eg_batch_tuning tuning{};
+    DevBuf consts;  // BConst
     DevBuf qs, items, citems, tables, metas;  // metas: per-query meta + counts + status + queue
     DevBuf ptiles, pqs, hist, skeys, svals;     // the partition pass (radix_bits > 0)
     int n_items = 0, n_citems = 0, n_ptiles = 0, n_pq = 0;
@@ -486,6 +639,17 @@ void batch_default_tuning(eg_batch_tuning* t)
     t->lds_max_bound_log2 = 11;
     t->blocks_per_cu = 1;
     t->radix_bits = 12;
+}
+
+// The aggregation kernel for the plan's key and value widths.
+auto agg_kernel(const BatchPlan& p) -> decltype(&batch_agg_kernel<4, 0>)
+{
+    const int vb = p.nv == 0 ? 0 : p.vbytes == 4 || p.vbytes == 8 ? p.vbytes : -1;
+    if (p.kb == 4)
+        return vb == 0 ? batch_agg_kernel<4, 0> : vb == 4 ? batch_agg_kernel<4, 4> : vb == 8 ? batch_agg_kernel<4, 8>
+             : batch_agg_kernel<4, -1>;
+    return vb == 0 ? batch_agg_kernel<8, 0> : vb == 4 ? batch_agg_kernel<8, 4> : vb == 8 ? batch_agg_kernel<8, 8>
+         : batch_agg_kernel<8, -1>;
 }
 
 BatchPlan* batch_plan_create(const eg_batch_query* queries, int64_t nq, int32_t key_type, int32_t val_type,
@@ -522,6 +686,14 @@ BatchPlan* batch_plan_create(const eg_batch_query* queries, int64_t nq, int32_t 
     p->nv = plan.spec.nvcols;
     p->vbytes = uses_vals ? type_size(val_type) : 8;
     p->W = table_words_per_slot(plan.spec.nops);
+    if (plan.spec.nops > EG_BATCH_MAX_AGGS) raise(EG_ERR_UNSUPPORTED, "too many aggregation states for a batch");
+    p->ops.codes = ~0u;
+    p->ops.conv = uses_vals ? plan.spec.cols[0].conv : (int32_t)CONV_RAW;
+    for (int a = 0; a < plan.spec.nops; ++a) {
+        const int32_t code = plan.spec.ops[a].code;
+        p->ops.codes = (p->ops.codes & ~(0xffu << (8 * a))) | (uint32_t)code << (8 * a);
+        p->ops.has_any |= op_class(code) == CLS_XCHG ? 1 : 0;
+    }
     p->bo.nouts = (int32_t)plan.outs.size();
     p->bo.key_bytes = plan.key.bytes;
     for (size_t j = 0; j < plan.outs.size(); ++j) {
@@ -554,7 +726,7 @@ BatchPlan* batch_plan_create(const eg_batch_query* queries, int64_t nq, int32_t 
     std::vector<uint64_t> offs((size_t)nq);
     uint64_t words = 0;
     int64_t hist_entries = 0, scratch_rows = 0;
-    constexpr uint64_t kCompactRange = 1u << 16;
+    constexpr uint64_t kCompactRange = 4 * 256 * kCompactSlots;  // four rounds a workgroup
     for (int64_t i = 0; i < nq; ++i) {
         const eg_batch_query& u = queries[i];
         if (u.rows < 0 || u.capacity < 0) raise(EG_ERR_INVALID, "negative batch query size");
@@ -595,12 +767,13 @@ BatchPlan* batch_plan_create(const eg_batch_query* queries, int64_t nq, int32_t 
             hpq.push_back((int32_t)i);
             for (int64_t t = 0; t < q.ntiles; ++t) htiles.push_back(BPTile{(int32_t)i, (int32_t)t});
             for (int64_t d = 0; d < ((int64_t)1 << q.pbits); ++d) {
-                hitems.push_back(BItem{(int32_t)i, 1, d, d + 1});
+                hitems.push_back(BItem{(int32_t)i, kItemPart, d, d + 1});
                 item_rows.push_back(u.rows >> q.pbits);
             }
         } else {
             for (int64_t b = 0; b < u.rows; b += tile) {
-                hitems.push_back(BItem{(int32_t)i, 0, b, std::min(u.rows, b + tile)});
+                const int32_t kind = q.use_lds && u.rows <= tile ? kItemWhole : kItemRows;
+                hitems.push_back(BItem{(int32_t)i, kind, b, std::min(u.rows, b + tile)});
                 item_rows.push_back(std::min(u.rows, b + tile) - b);
             }
         }
@@ -653,23 +826,24 @@ BatchPlan* batch_plan_create(const eg_batch_query* queries, int64_t nq, int32_t 
         EG_HIP(hipMemcpyAsync(p->ptiles.get(), htiles.data(), htiles.size() * sizeof(BPTile), hipMemcpyHostToDevice, s));
         EG_HIP(hipMemcpyAsync(p->pqs.get(), hpq.data(), hpq.size() * sizeof(int32_t), hipMemcpyHostToDevice, s));
     }
+    const BConst hconst{p->spec, p->bo};
+    p->consts = DevBuf(sizeof(BConst), s);
+    EG_HIP(hipMemcpyAsync(p->consts.get(), &hconst, sizeof hconst, hipMemcpyHostToDevice, s));
     EG_HIP(hipStreamSynchronize(s));  // the host vectors go out of scope
 
     p->grid = di.num_cus * T.blocks_per_cu;
     // raise the kernel's LDS limit now: no attribute calls during graph capture
-    const void* kern = p->kb == 4 ? (const void*)batch_agg_kernel<4, 1> : (const void*)batch_agg_kernel<8, 1>;
-    if (enable_dynamic_lds(kern) < p->lds) raise(EG_ERR_UNSUPPORTED, "batch LDS table too large");
+    if (enable_dynamic_lds((const void*)agg_kernel(*p)) < p->lds) raise(EG_ERR_UNSUPPORTED, "batch LDS table too large");
     return p.release();
 }
 
-template <int KB, int NV>
 void launch_batch_agg(BatchPlan& p, hipStream_t s)
 {
-    auto kern = batch_agg_kernel<KB, NV>;
-    hipLaunchKernelGGL(kern, dim3(p.grid), dim3(kBatchBlock), p.lds, s, p.qs.get<BQuery>(), p.items.get<BItem>(),
-                       p.n_items, p.next_item, p.metas.get<unsigned long long>(), p.spec, is_signed_int(p.key_type) ? 1 : 0,
-                       p.vbytes, p.W, p.tuning.lds_slots_log2, 16, 8, (const uint32_t*)p.hist.get<uint32_t>(),
-                       (const void*)p.skeys.get(), (const void*)p.svals.get(), p.counts, p.qstatus, p.bo);
+    hipLaunchKernelGGL(agg_kernel(p), dim3(p.grid), dim3(kBatchBlock), p.lds, s, p.qs.get<BQuery>(), p.items.get<BItem>(),
+                       p.n_items, p.next_item, p.metas.get<unsigned long long>(), (const BConst*)p.consts.get<BConst>(),
+                       p.ops, (int)p.spec.nops, is_signed_int(p.key_type) ? 1 : 0, p.vbytes, p.W,
+                       p.tuning.lds_slots_log2, 16, 8, (const uint32_t*)p.hist.get<uint32_t>(),
+                       (const void*)p.skeys.get(), (const void*)p.svals.get(), p.counts, p.qstatus);
     EG_LAUNCH_CHECK();
 }
 
@@ -707,12 +881,11 @@ void batch_run(BatchPlan& p, hipStream_t s)
     }
     {
         KernelTimer timer("batch_agg", s);
-        if (p.kb == 4) launch_batch_agg<4, 1>(p, s);
-        else launch_batch_agg<8, 1>(p, s);
+        launch_batch_agg(p, s);
     }
     KernelTimer timer("batch_compact", s);
     hipLaunchKernelGGL(batch_compact_kernel, dim3(p.n_citems), dim3(256), 0, s, p.qs.get<BQuery>(), p.citems.get<BCItem>(),
-                       p.metas.get<unsigned long long>(), p.counts, p.qstatus, p.bo, p.W);
+                       p.metas.get<unsigned long long>(), p.counts, p.qstatus, (const BConst*)p.consts.get<BConst>(), p.W);
     EG_LAUNCH_CHECK();
 }
 

@@ -26,3 +26,50 @@ def test_sort_strategy_keys_sharing_low_bits(n, dtype, shift, low, minimum):
     exp = sorted_by_key(O.groupby(keys, [vals], reqs))
     for fn in (G.sort_groupby, G.sort_groupby_gfur):
         assert_same(run(fn, keys, [vals], reqs), exp)
+
+
+@pytest.mark.parametrize("ktype", [np.int32, np.int64])
+@pytest.mark.parametrize("vtype,kinds", [
+    (np.int64, (A.SUM, A.MIN, A.MAX, A.COUNT_ALL)), (np.float32, (A.SUM, A.MIN, A.MAX)), (np.uint32, (A.MAX, A.MIN)),
+    (np.int16, (A.SUM, A.MIN)), (np.float64, (A.MAX, A.SUM)), (None, (A.COUNT_ALL,)), (np.int32, (A.ANY, A.COUNT_ALL))])
+def test_batch_value_widths_hot_keys_and_full_tables(ktype, vtype, kinds):
+    """One batch of every way through the aggregation kernel: whole-query,
+    row-range and partition items; 1/4/8-byte and no values; a key most rows
+    hold; more groups than the LDS table has slots; the empty-slot key; row
+    counts around a step."""
+    rng = np.random.default_rng(11)
+    info = np.iinfo(ktype)
+    shapes = [(1, 1), (63, 5), (4096, 40), (4097, 4097), (40_000, 300), (70_001, 3000), (200_003, 20_000)]
+    queries, datas, keep = [], [], []
+    for n, d in shapes:
+        keys = rng.integers(0, d, n).astype(ktype)
+        keys[rng.random(n) < 0.5] = keys[0]          # a hot key
+        if n > 10:
+            keys[5], keys[6] = info.min, info.max    # INT_MIN encodes to the empty slot word
+        vals = None
+        if vtype is not None:
+            vals = (rng.integers(-500, 500, n) if np.dtype(vtype).kind != "u" else rng.integers(0, 1000, n)).astype(vtype)
+            if kinds[0] == A.ANY:
+                vals = (keys.astype(np.int64) % 1000).astype(vtype)  # one value per key
+        g = len(np.unique(keys))
+        outs = [G.make_column(G.to_type_id(ktype), g)]
+        for k in kinds:
+            outs.append(G.make_column(G.agg_output_data_type(k, G.to_type_id(vtype or np.int64)), g))
+        kc = G.make_column_from_host(keys)
+        vc = None if vals is None else G.make_column_from_host(vals)
+        keep += [kc, vc]
+        queries.append(G.batch_query(kc, vc, g, outs[0], outs[1:]))
+        datas.append((keys, vals, outs))
+    reqs = [(-1 if k == A.COUNT_ALL else 0, k) for k in kinds]
+    for tuning in (G.batch_tuning(tile_rows_log2=16, lds_slots_log2=9, lds_max_bound_log2=12, blocks_per_cu=2, radix_bits=10),
+                   G.batch_tuning(tile_rows_log2=10, lds_slots_log2=6, lds_max_bound_log2=8, blocks_per_cu=1, radix_bits=0)):
+        plan = G.batch_plan(queries, G.to_type_id(ktype), G.to_type_id(vtype or np.int64), reqs, tuning)
+        for launch in (plan.run, plan.graph_launch, plan.graph_launch):
+            launch()
+            ng, st = plan.results()
+            assert not st.any()
+            for (keys, vals, outs), g in zip(datas, ng):
+                exp = sorted_by_key(O.groupby(keys, [] if vals is None else [vals], reqs))
+                got = sorted_by_key([o.to_numpy()[:g] for o in outs])
+                assert_same(got, exp, 1e-5 if vtype == np.float32 else 1e-9)
+        plan.free()
