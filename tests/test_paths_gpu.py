@@ -73,3 +73,20 @@ def test_batch_value_widths_hot_keys_and_full_tables(ktype, vtype, kinds):
                 got = sorted_by_key([o.to_numpy()[:g] for o in outs])
                 assert_same(got, exp, 1e-5 if vtype == np.float32 else 1e-9)
         plan.free()
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64, np.uint16, np.uint32])
+@pytest.mark.parametrize("m", [4096, 4097, 6143, 6145, 12_289, 50_000])
+def test_dictionary_table_sizes_around_the_lds_limit_and_load(dtype, m):
+    """Dictionaries around the last LDS table, around the load at which the
+    HBM table doubles, with repeats, absent keys and the type's extremes."""
+    info = np.iinfo(dtype)
+    rng = np.random.default_rng(m)
+    pool = rng.integers(info.min, info.max, m, dtype=dtype, endpoint=True)
+    pool[0], pool[1] = info.min, info.max
+    pool[m // 2] = pool[m // 3]  # a repeated key: its first position counts
+    n = 4 * 2048 + 77
+    keys = np.where(rng.random(n) < 0.7, rng.choice(pool, n), rng.integers(info.min, info.max, n, dtype=dtype, endpoint=True)).astype(dtype)
+    kc, dc = G.make_column_from_host(keys), G.make_column_from_host(pool)
+    got = G.dictionary_encode_with_dict(kc, dc).to_numpy()
+    np.testing.assert_array_equal(got, O.dict_encode(keys, pool))
