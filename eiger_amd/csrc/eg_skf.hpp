@@ -32,7 +32,8 @@ struct FuseStage {
 };
 
 struct FusedKeys {
-    DevBuf fused;                  // rows x uint64 fused keys
+    DevBuf fused;                  // rows x fused keys of key_bytes
+    int key_bytes = 8;             // 4 when the fields take at most 32 bits
     int ncols = 0;
     int64_t rows = 0;
     int total_bits = 0;            // bits of the fused key

@@ -542,8 +542,14 @@ extern "C" int eg_jit_prefetch(int32_t key_type, const int32_t* val_types, int64
         set_outspec(plan, nullptr, none, os);
         lds::with_vlayout(plan.spec, true, [&](auto vl) {
             const std::string name = jit::vlayout_name<decltype(vl)>();
-            n += jit::prefetch(jit::Kind::HASH_AGG, plan.key.bytes, name, plan.spec, a) ? 1 : 0;
-            n += jit::prefetch(jit::Kind::PART_AGG, plan.key.bytes, name, plan.spec, a, &os) ? 1 : 0;
+            auto queue = [&](int kb) {
+                n += jit::prefetch(jit::Kind::HASH_AGG, kb, name, plan.spec, a) ? 1 : 0;
+                n += jit::prefetch(jit::Kind::PART_AGG, kb, name, plan.spec, a, &os) ? 1 : 0;
+            };
+            queue(plan.key.bytes);
+            // UINT64 is what several key columns fuse into, or UINT32 where
+            // their fields take at most 32 bits: ready for either
+            if (key_type == EG_UINT64) queue(4);
         });
         if (queued) *queued = n;
     });

@@ -35,6 +35,7 @@
 #include "eg_internal.hpp"
 #include "eg_jit.hpp"
 #include "eg_lds_table.hpp"
+#include "eg_part_launch.hpp"
 #include "eg_radix.hpp"
 
 namespace eg {
@@ -83,19 +84,6 @@ using agg::kPBMax;
 using agg::Unit;
 
 using agg::OutClaims;
-
-// Eight waves per SIMD: two 1024-thread workgroups per CU, which the LDS
-// table is sized for (without the bound the compiler's scalar registers
-// alone leave room for only one).
-template <int KB, class VL, bool GATHER>
-__global__ __launch_bounds__(kPBMax, 8) void part_agg_kernel(KeyDesc key, AggSpec spec, const int64_t* perm,
-                                                       const Unit* units, GTable gt, OutSpec os,
-                                                       OutClaims claims, int64_t capacity,
-                                                       int cr, int probe, int peel_min)
-{
-    agg::part_agg<KB, VL, dev::RtOps, GATHER>(key, spec, perm, units, gt, os, claims, capacity, cr, probe,
-                                              peel_min);
-}
 
 template <int KB>
 __device__ __forceinline__ uint32_t pid_of(uint64_t raw, uint32_t mask)
@@ -188,39 +176,6 @@ int ceil_log2(int64_t x)
     int b = 0;
     while (((int64_t)1 << b) < x) ++b;
     return b;
-}
-
-template <int KB, bool GATHER>
-void launch_part_agg(const KeyDesc& key, const AggSpec& spec, const int64_t* perm, const Unit* units, int nunits,
-                     const GTable& gt, const OutSpec& os, const OutClaims& claims, int64_t capacity, int cr,
-                     size_t lds, int block, int64_t rows, hipStream_t s)
-{
-    with_vlayout(spec, true, [&](auto vl) {
-        using VL = decltype(vl);
-        auto kern = part_agg_kernel<KB, VL, GATHER>;
-        if (enable_dynamic_lds((const void*)kern) < lds) raise(EG_ERR_UNSUPPORTED, "partition LDS table too large");
-        KernelTimer timer("partition_agg", s);
-        int probe = 16, peel_min = default_peel_min();  // probe: buckets of four slots
-        // the kernel with this request's ops compiled in, once it is available
-        const jit::Kind kind = GATHER ? jit::Kind::PART_AGG_GATHER : jit::Kind::PART_AGG;
-        if (hipFunction_t f = jit::lookup(kind, KB, jit::vlayout_name<VL>(), spec, rows, &os)) {
-            KeyDesc a_key = key;
-            AggSpec a_spec = spec;
-            const int64_t* a_perm = perm;
-            const Unit* a_units = units;
-            GTable a_gt = gt;
-            OutSpec a_os = os;
-            OutClaims a_claims = claims;
-            int64_t a_cap = capacity;
-            int a_cr = cr;
-            void* args[] = {&a_key, &a_spec, &a_perm, &a_units, &a_gt, &a_os, &a_claims, &a_cap, &a_cr,
-                            &probe, &peel_min};
-            if (jit::launch(f, (unsigned)nunits, (unsigned)block, lds, s, args)) return;
-        }
-        hipLaunchKernelGGL(kern, dim3(nunits), dim3(block), lds, s, key, spec, perm, units, gt, os, claims, capacity,
-                           cr, probe, peel_min);
-        EG_LAUNCH_CHECK();
-    });
 }
 
 template <int KB>
@@ -345,12 +300,15 @@ Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream
         EG_LAUNCH_CHECK();
     }
     // Rows per unit: a partition is split when it is much larger than the
-    // average (skew), or when there are too few partitions to occupy every CU,
-    // since a split partition's groups merge through the HBM table with
-    // atomics instead of being written straight out.
+    // average (skew), or when there are too few partitions to occupy every CU
+    // twice, since a split partition's groups merge through the HBM table with
+    // atomics instead of being written straight out.  (Splitting at
+    // n / (4 CUs) also with 1024 partitions cut a quarter of them in two: 25M
+    // rows in 700k groups, unit kernel and compaction 289 + 64 us.)
     const int64_t avg_rows = (n + P - 1) / P;
     const int64_t balance = std::max<int64_t>(1, n / (4 * (int64_t)di.num_cus));
-    const int64_t slice = std::max<int64_t>({(int64_t)tune.block * 16, 8 * per_part, std::min(4 * avg_rows, balance)});
+    const int64_t fair = P >= 2 * (int64_t)di.num_cus ? 4 * avg_rows : std::min(4 * avg_rows, balance);
+    const int64_t slice = std::max<int64_t>({(int64_t)tune.block * 16, 8 * per_part, fair});
     // units built on the device; 16 bytes (unit and sliced-partition counts)
     // come back instead of the boundaries, and no unit list goes up
     const int64_t max_units = P + n / slice + 1;

@@ -48,24 +48,57 @@ struct FuseArgs {
     uint64_t mask[kMaxFuseItems];
 };
 
-__global__ __launch_bounds__(256) void fuse_keys_kernel(FuseArgs a, int64_t n, uint64_t* __restrict__ fused)
+// Four rows a thread: a column's width is switched on once per four
+// independent loads.  T: 4-byte fused keys where the fields take at most 32
+// bits, so everything after (partition passes, tables) moves half the key.
+template <typename T>
+__global__ __launch_bounds__(256) void fuse_keys_kernel(FuseArgs a, int64_t n, T* __restrict__ fused)
 {
+    constexpr int U = 4;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        uint64_t f = 0;
-        for (int c = 0; c < a.nitems; ++c) {
-            const uint64_t t = twiddle_bits(dev::load_raw(a.data[c], a.bytes[c], i), a.type[c], a.bytes[c]);
-            f |= (t - a.min[c]) << a.shift[c];
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += U * stride) {
+        uint64_t f[U], raw[U];
+        int64_t r[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            f[u] = 0;
+            r[u] = i + u * stride < n ? i + u * stride : i;
         }
-        fused[i] = f;
+        for (int c = 0; c < a.nitems; ++c) {
+            switch (a.bytes[c]) {  // uniform
+            case 1:
+#pragma unroll
+                for (int u = 0; u < U; ++u) raw[u] = ((const uint8_t*)a.data[c])[r[u]];
+                break;
+            case 2:
+#pragma unroll
+                for (int u = 0; u < U; ++u) raw[u] = ((const uint16_t*)a.data[c])[r[u]];
+                break;
+            case 4:
+#pragma unroll
+                for (int u = 0; u < U; ++u) raw[u] = ((const uint32_t*)a.data[c])[r[u]];
+                break;
+            default:
+#pragma unroll
+                for (int u = 0; u < U; ++u) raw[u] = ((const uint64_t*)a.data[c])[r[u]];
+                break;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) f[u] |= (twiddle_bits(raw[u], a.type[c], a.bytes[c]) - a.min[c]) << a.shift[c];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (i + u * stride < n) fused[r[u]] = (T)f[u];
     }
 }
 
-__global__ __launch_bounds__(256) void unfuse_keys_kernel(FuseArgs a, int64_t n, const uint64_t* __restrict__ fused)
+// key_bytes: width of `fused` (4 or 8)
+__global__ __launch_bounds__(256) void unfuse_keys_kernel(FuseArgs a, int64_t n, const void* __restrict__ fused,
+                                                          int key_bytes)
 {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const uint64_t f = fused[i];
+        const uint64_t f = key_bytes == 4 ? (uint64_t)((const uint32_t*)fused)[i] : ((const uint64_t*)fused)[i];
         for (int c = 0; c < a.nitems; ++c) {
             uint64_t x = (f >> a.shift[c]) & a.mask[c];
             if (a.table[c]) x = a.table[c][x];
@@ -252,13 +285,13 @@ void fuse_keys(const ViewIn* keys, int64_t ncols, hipStream_t s, FusedKeys& f)
     std::vector<DevBuf> col_ranks((size_t)ncols);  // dense ranks of ranked columns
     // Assigns the stage's shifts (first item in the most significant bits,
     // zero-width items none) and fuses its items for every row.
-    auto run_stage = [&](FuseStage& st, int width) {
+    auto run_stage = [&](FuseStage& st, int width, bool narrow) {
         int shift = width;
         for (int j = 0; j < st.nitems; ++j) {
             shift -= st.items[j].bits;
             st.items[j].shift = st.items[j].bits > 0 ? shift : 0;
         }
-        DevBuf out((size_t)std::max<int64_t>(n, 1) * 8, s);
+        DevBuf out((size_t)std::max<int64_t>(n, 1) * (narrow ? 4 : 8), s);
         if (n > 0) {
             FuseArgs a{};
             a.nitems = st.nitems;
@@ -277,8 +310,12 @@ void fuse_keys(const ViewIn* keys, int64_t ncols, hipStream_t s, FusedKeys& f)
                     a.min[j] = f.min[it.src];
                 }
             }
-            hipLaunchKernelGGL(fuse_keys_kernel, dim3((unsigned)grid_of(n)), dim3(256), 0, s, a, n,
-                               out.get<uint64_t>());
+            if (narrow)
+                hipLaunchKernelGGL(fuse_keys_kernel<uint32_t>, dim3((unsigned)grid_of(n)), dim3(256), 0, s, a, n,
+                                   out.get<uint32_t>());
+            else
+                hipLaunchKernelGGL(fuse_keys_kernel<uint64_t>, dim3((unsigned)grid_of(n)), dim3(256), 0, s, a, n,
+                                   out.get<uint64_t>());
             EG_LAUNCH_CHECK();
         }
         return out;
@@ -292,7 +329,7 @@ void fuse_keys(const ViewIn* keys, int64_t ncols, hipStream_t s, FusedKeys& f)
         it.bits = f.bits[c];
         if (width + it.bits > 64 || cur.nitems == kMaxFuseItems) {
             // the columns so far become the dense rank of their fused value
-            DevBuf v = run_stage(cur, width);
+            DevBuf v = run_stage(cur, width, false);
             const int64_t nd = dense_ranks(v.get<uint64_t>(), n, width, s, prev_ranks, cur.table);
             f.stages.push_back(std::move(cur));
             cur = FuseStage{};
@@ -304,7 +341,7 @@ void fuse_keys(const ViewIn* keys, int64_t ncols, hipStream_t s, FusedKeys& f)
             if (width + it.bits > 64) {  // and this column its own dense rank
                 FuseStage one;
                 one.items[one.nitems++] = it;
-                DevBuf w = run_stage(one, it.bits);
+                DevBuf w = run_stage(one, it.bits, false);
                 const int64_t ndc =
                     dense_ranks(w.get<uint64_t>(), n, it.bits, s, col_ranks[(size_t)c], f.col_table[(size_t)c]);
                 it.ranked = 1;
@@ -315,7 +352,8 @@ void fuse_keys(const ViewIn* keys, int64_t ncols, hipStream_t s, FusedKeys& f)
         width += it.bits;
     }
     f.total_bits = width;
-    f.fused = run_stage(cur, width);
+    f.key_bytes = width <= 32 ? 4 : 8;
+    f.fused = run_stage(cur, width, f.key_bytes == 4);
     f.stages.push_back(std::move(cur));
 }
 
@@ -353,7 +391,7 @@ std::vector<DevBuf> unfuse_keys(const FusedKeys& f, const void* fused, int64_t g
             }
         }
         hipLaunchKernelGGL(unfuse_keys_kernel, dim3((unsigned)grid_of(groups)), dim3(256), 0, s, a, groups,
-                           (const uint64_t*)cur);
+                           cur, st + 1 == (int)f.stages.size() ? f.key_bytes : 8);
         EG_LAUNCH_CHECK();
         cur_buf = std::move(prev);
         cur = cur_buf.get();

@@ -90,3 +90,36 @@ def test_dictionary_table_sizes_around_the_lds_limit_and_load(dtype, m):
     kc, dc = G.make_column_from_host(keys), G.make_column_from_host(pool)
     got = G.dictionary_encode_with_dict(kc, dc).to_numpy()
     np.testing.assert_array_equal(got, O.dict_encode(keys, pool))
+
+
+@pytest.mark.parametrize("bits", [(16, 16), (17, 16), (1, 31), (32,), (33,), (8, 8, 8, 8)])
+@pytest.mark.parametrize("algo", ["AUTO_ALGO", "HASH", "SORT", "PARTITION"])
+def test_fused_keys_around_32_bits(bits, algo):
+    """Key columns whose fields take just under, exactly and just over 32
+    bits: the fused key is 4 or 8 bytes wide; the extreme tuples are there."""
+    rng = np.random.default_rng(sum(bits))
+    n = 9001
+    cols = []
+    for b in bits:
+        c = rng.integers(0, 1 << b, n, dtype=np.int64)
+        c[0], c[1] = 0, (1 << b) - 1
+        cols.append(c - (1 << (b - 1)))
+    if len(cols) == 1:
+        cols.append(np.full(n, -7, np.int16))  # a constant column: no bits
+    for c in cols:
+        c[2:200] = c[200:398]  # some repeated tuples
+    vals = rng.integers(-100, 100, n).astype(np.int32)
+    kc = [G.make_column_from_host(c) for c in cols]
+    t = G.groupby(kc, [G.make_column_from_host(vals)], [(0, A.SUM), (-1, A.COUNT_ALL)],
+                  G.groupby_hint(groupby_algo=G.groupby_algo[algo], enable_skf=True))
+    got = t.to_numpy()
+    exp = {}
+    for i, tup in enumerate(zip(*[c.tolist() for c in cols])):
+        s, k = exp.get(tup, (0, 0))
+        exp[tup] = (s + int(vals[i]), k + 1)
+    rows = list(zip(*[g.tolist() for g in got[:len(cols)]]))
+    assert len(rows) == len(exp)
+    for r, s, k in zip(rows, got[-2].tolist(), got[-1].tolist()):
+        assert exp[r] == (s, k)
+    if algo == "SORT":
+        assert rows == sorted(rows)
