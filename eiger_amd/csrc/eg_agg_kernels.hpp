@@ -27,41 +27,72 @@ using namespace lds;
 template <int NV>
 constexpr int max_block() { return NV <= 2 ? 1024 : 512; }
 
-// Merges the replicas of the block's LDS table and adds every group to the
-// HBM table.
+// Merges replicas 1..R-1 of the block's LDS table into replica 0.
+template <class OPS, int KB>
+__device__ __forceinline__ void merge_replicas(LdsTable<KB>& tab, const GTable& gt, const KeyDesc& key,
+                                               const AggSpec& spec, int rep_log2, int r_mask, uint32_t& ins)
+{
+    using KT = typename LdsKey<KB>::T;
+    if (rep_log2 == 0) return;
+    for (int idx = threadIdx.x; idx < tab.T; idx += blockDim.x) {
+        const int r = idx & r_mask;
+        if (r == 0) continue;
+        const int s = idx >> rep_log2;
+        int dst;
+        KT kw = 0;
+        if (s == tab.cr) {
+            if (tab.side[r] == 0ull) continue;
+            dst = tab.find((KT)0, 0, 1);
+        } else {
+            kw = tab.keys[idx];
+            if (kw == 0) continue;
+            dst = tab.find(kw, 0, tab.cr);
+        }
+        auto src = [&](int a) { return tab.st[(size_t)a * tab.T + idx]; };
+        if (dst >= 0) {
+            dev::merge_states<OPS>(spec, [&](int a) { return &tab.st[(size_t)a * tab.T + dst]; }, src);
+        } else {
+            // replica 0 is full: merge this slot straight into HBM
+            unsigned long long* g = gt_slot(gt, lds_to_enc64<KB>(kw, key.is_signed), ins);
+            if (g) dev::merge_states<OPS>(spec, [&](int a) { return g + 1 + a; }, src);
+        }
+    }
+    __syncthreads();
+}
+
+// Ends a block's aggregation: its groups go to the HBM table with atomics,
+// or (priv) its table is stored as it stands for table_merge to combine.
+// Every block of a large grid holds the same groups, so the atomics of all
+// blocks meet on the same few lines: 256 blocks of 1024 groups and two states
+// took 250 us, the stored tables and their merge 25.
+// Words of a stored table: cr + 1 keys (64-bit encoding, 0 = empty; the side
+// slot last: its encoding, or 1 where that is 0), then cr + 1 states per op.
 template <class OPS, int KB>
 __device__ __forceinline__ void flush_lds(LdsTable<KB>& tab, const GTable& gt, const KeyDesc& key, const AggSpec& spec,
-                          int rep_log2, int r_mask, uint32_t& ins)
+                          int rep_log2, int r_mask, uint32_t& ins, unsigned long long* priv)
 {
     using KT = typename LdsKey<KB>::T;
     __syncthreads();
-    // merge replicas 1..R-1 into replica 0 (LDS atomics)
-    const int R = 1 << rep_log2;
-    if (R > 1) {
-        for (int idx = threadIdx.x; idx < tab.T; idx += blockDim.x) {
-            const int r = idx & r_mask;
-            if (r == 0) continue;
-            const int s = idx >> rep_log2;
-            int dst;
-            KT kw = 0;
+    merge_replicas<OPS>(tab, gt, key, spec, rep_log2, r_mask, ins);
+    if (priv) {
+        const int nops = OPS::n(spec);
+        unsigned long long* out = priv + (size_t)blockIdx.x * (size_t)(1 + nops) * (tab.cr + 1);
+        for (int s = threadIdx.x; s <= tab.cr; s += blockDim.x) {
+            const int idx = s << rep_log2;
+            unsigned long long e;
             if (s == tab.cr) {
-                if (tab.side[r] == 0ull) continue;
-                dst = tab.find((KT)0, 0, 1);
+                e = tab.side[0] == 0ull ? 0ull : (KB == 8 ? 1ull : lds_to_enc64<KB>((KT)0, key.is_signed));
             } else {
-                kw = tab.keys[idx];
-                if (kw == 0) continue;
-                dst = tab.find(kw, 0, tab.cr);
+                const KT kw = tab.keys[idx];
+                e = kw == 0 ? 0ull : lds_to_enc64<KB>(kw, key.is_signed);
             }
-            auto src = [&](int a) { return tab.st[(size_t)a * tab.T + idx]; };
-            if (dst >= 0) {
-                dev::merge_states<OPS>(spec, [&](int a) { return &tab.st[(size_t)a * tab.T + dst]; }, src);
-            } else {
-                // replica 0 is full: merge this slot straight into HBM
-                unsigned long long* g = gt_slot(gt, lds_to_enc64<KB>(kw, key.is_signed), ins);
-                if (g) dev::merge_states<OPS>(spec, [&](int a) { return g + 1 + a; }, src);
-            }
+            out[s] = e;
+            if (e == 0ull) continue;  // the states of an empty slot are never read
+            dev::for_each_op<OPS>(spec, [&](auto a) {
+                out[(size_t)(1 + (int)a) * (tab.cr + 1) + s] = tab.st[(size_t)(int)a * tab.T + idx];
+            });
         }
-        __syncthreads();
+        return;
     }
     // flush replica 0 into the HBM table
     for (int s = threadIdx.x; s <= tab.cr; s += blockDim.x) {
@@ -78,6 +109,59 @@ __device__ __forceinline__ void flush_lds(LdsTable<KB>& tab, const GTable& gt, c
         if (!g) continue;
         dev::merge_states<OPS>(spec, [&](int a) { return g + 1 + a; }, [&](int a) { return tab.st[(size_t)a * tab.T + idx]; });
     }
+}
+
+// Combines the tables that `nb` blocks stored (see flush_lds): this block
+// takes slots [blockIdx.x * kMergeSlots, + kMergeSlots) of every one, groups
+// them in an LDS table of 8-byte encoded keys, and adds the result to the HBM
+// table.  A key sits at or after its home slot, so its copies fall into one
+// block's range, or few; the few meet in the HBM table.
+constexpr int kMergeSlots = 8;   // 64-byte runs of a stored table, a block per range
+constexpr int kMergeCr = 64;     // LDS slots: the range's keys and displaced ones
+constexpr int kMergeBlock = 512;
+
+__device__ __forceinline__ void table_merge(const unsigned long long* priv, int nb, int cr, const AggSpec& spec,
+                                            const GTable& gt, bool key8)
+{
+    extern __shared__ __align__(16) unsigned long long smem[];
+    const int nops = spec.nops;
+    LdsTable<8, true> tab(smem, nops, kMergeCr, 0);
+    const int words = LdsTable<8>::words(nops, kMergeCr, 0);
+    for (int i = threadIdx.x; i < words; i += blockDim.x) smem[i] = 0ull;
+    __syncthreads();
+    const size_t tw = (size_t)(1 + nops) * (cr + 1);
+    const int s0 = blockIdx.x * kMergeSlots;
+    const int ns = min(kMergeSlots, cr + 1 - s0);
+    uint32_t ins = 0;
+    for (int i = threadIdx.x; i < nb * kMergeSlots; i += blockDim.x) {
+        const int off = i % kMergeSlots;
+        if (off >= ns) continue;
+        const unsigned long long* t = priv + (size_t)(i / kMergeSlots) * tw + s0 + off;
+        unsigned long long e = t[0];
+        if (e == 0ull) continue;
+        if (key8 && s0 + off == cr) e = 0ull;  // the side slot of 8-byte keys
+        auto src = [&](int a) { return t[(size_t)(1 + a) * (cr + 1)]; };
+        const int slot = tab.find(e, 0, kMergeCr);
+        if (slot >= 0) {
+            dev::merge_states<dev::RtOps>(spec, [&](int a) { return &tab.st[(size_t)a * tab.T + slot]; }, src);
+        } else {
+            unsigned long long* g = gt_slot(gt, e, ins);
+            if (g) dev::merge_states<dev::RtOps>(spec, [&](int a) { return g + 1 + a; }, src);
+        }
+    }
+    __syncthreads();
+    for (int s = threadIdx.x; s <= tab.cr; s += blockDim.x) {
+        unsigned long long e = 0ull;
+        if (s < tab.cr) {
+            e = tab.keys[s];
+            if (e == 0ull) continue;
+        } else if (tab.side[0] == 0ull) {
+            continue;
+        }
+        unsigned long long* g = gt_slot(gt, e, ins);
+        if (g) dev::merge_states<dev::RtOps>(spec, [&](int a) { return g + 1 + a; }, [&](int a) { return tab.st[(size_t)a * tab.T + s]; });
+    }
+    gt_count_inserts(gt, ins);
 }
 
 // Whether a fixed op list can keep per-lane partial states of one group in
@@ -108,7 +192,8 @@ constexpr int kPrivLanes = 8;
 
 template <int KB, class VL, class OPS>
 __device__ __forceinline__ void hash_agg(const KeyDesc& key, int64_t n, const AggSpec& spec, const GTable& gt,
-                                         int cr, int rep_log2, int probe_limit, int peel_min)
+                                         int cr, int rep_log2, int probe_limit, int peel_min,
+                                         unsigned long long* priv)
 {
     constexpr int NV = VL::NV > 0 ? VL::NV : 1;
     extern __shared__ __align__(16) unsigned long long smem[];
@@ -274,7 +359,7 @@ __device__ __forceinline__ void hash_agg(const KeyDesc& key, int64_t n, const Ag
         const bool sp = lds_row<OPS, KB, NV>(tab, use_lds, r_mask, lane, key, spec, kraw, cv, valid, probe_limit, peel_min, hot);
         if (__ballot(sp) != 0ull) hbm_rows<OPS, KB, NV>(gt, key, spec, sp, kraw, cv, hbm_peel, ins, hot);
     }
-    if (use_lds) flush_lds<OPS>(tab, gt, key, spec, rep_log2, r_mask, ins);
+    if (use_lds) flush_lds<OPS>(tab, gt, key, spec, rep_log2, r_mask, ins, priv);
     gt_count_inserts(gt, ins);
 }
 

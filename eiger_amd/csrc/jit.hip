@@ -268,9 +268,9 @@ std::string make_source(Kind kind, int kb, const std::string& vl, const AggSpec&
     if (kind == Kind::HASH_AGG) {
         o << "extern \"C\" __global__ __launch_bounds__(eg::agg::max_block<JitVL::NV>()) void eg_jit_hash_agg("
              "eg::KeyDesc key, int64_t n, eg::AggSpec spec, eg::GTable gt, int cr, int rep_log2, "
-             "int probe_limit, int peel_min)\n{\n"
+             "int probe_limit, int peel_min, unsigned long long* priv)\n{\n"
           << "    eg::agg::hash_agg<" << kb
-          << ", JitVL, JitOps>(key, n, spec, gt, cr, rep_log2, probe_limit, peel_min);\n}\n";
+          << ", JitVL, JitOps>(key, n, spec, gt, cr, rep_log2, probe_limit, peel_min, priv);\n}\n";
     } else {
         o << "extern \"C\" __global__ __launch_bounds__(eg::agg::kPBMax, 8) void eg_jit_part_agg(eg::KeyDesc key, "
              "eg::AggSpec spec, const int64_t* perm, const eg::agg::Unit* units, eg::GTable gt, eg::OutSpec os, "

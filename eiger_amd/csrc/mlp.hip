@@ -592,26 +592,32 @@ LoadedModel& loaded_model()
 // (~0.08 ms, one synchronisation) would cost more than any choice saves.
 constexpr int64_t kSmallRows = (int64_t)1 << 17;
 
+// Group counts up to which an input goes to hash whatever the class scores:
+// its tables then fit one workgroup's LDS, and a streaming pass with one merge
+// of the workgroups' tables beats radix passes.  2^24 rows and more: the
+// fastest for all such queries of the training and held-out traces (estimate
+// <= 2048).  Below: half of that, which leaves the bound made of an estimate
+// (2.5x) inside the LDS table for up to ten states; 2^20 rows in 1024 groups
+// 62 us by hash, 132 by partition.
+double hash_card(int64_t rows) { return rows >= ((int64_t)1 << 24) ? 2048.0 : 1280.0; }
+
 // Strategy from the model's outputs o[0..3] (class scores of hash / sort /
-// partition, log2 group count / 32).  A large input whose estimated group
-// count fits one LDS table goes to hash: one streaming pass, where every other
-// strategy makes radix passes (in the training and held-out traces hash was
-// the fastest for all such queries: rows >= 2^24, estimate <= 2048).
+// partition, log2 group count / 32), after hash_card's rule.
 int algo_of(const float* o, int64_t rows)
 {
     if (rows < kSmallRows) return EG_ALGO_HASH;
     const double card = std::exp2(std::min(62.0, std::max(0.0, (double)o[3] * 32.0)));
-    if (rows >= ((int64_t)1 << 24) && card <= 2048.0) return EG_ALGO_HASH;
+    if (card <= hash_card(rows)) return EG_ALGO_HASH;
     const int best = (o[1] > o[0] && o[1] >= o[2]) ? 1 : (o[2] > o[0] && o[2] > o[1]) ? 2 : 0;
     return best == 0 ? EG_ALGO_HASH : best == 1 ? EG_ALGO_SORT : EG_ALGO_PARTITION;
 }
 
-// A large input whose caller-given group bound already fits one LDS table
-// goes to hash without sampling: the bound caps the true group count, so
+// An input whose caller-given group bound already meets that rule goes to
+// hash without sampling: the bound caps the true group count, so
 // algo_of's rule would pick hash for any estimate the model could give.
 bool bound_picks_hash(int64_t rows, int64_t group_bound)
 {
-    return rows >= ((int64_t)1 << 24) && group_bound > 0 && group_bound <= 2048;
+    return rows >= kSmallRows && group_bound > 0 && (double)group_bound <= hash_card(rows);
 }
 
 // Learned strategy choice for one key column; false when no model is loaded.

@@ -123,3 +123,25 @@ def test_fused_keys_around_32_bits(bits, algo):
         assert exp[r] == (s, k)
     if algo == "SORT":
         assert rows == sorted(rows)
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64, np.uint64])
+@pytest.mark.parametrize("d", [1, 16, 1000, 7999, 16_400])
+@pytest.mark.parametrize("n", [16 * 4096, 200_003])
+def test_hash_tables_of_many_workgroups_merged(dtype, d, n):
+    """Grids of 16 workgroups and more store their LDS tables and merge them:
+    one group to twice the LDS slots, with the keys whose encodings are the
+    empty word, and undersized bounds."""
+    rng = np.random.default_rng(d)
+    info = np.iinfo(dtype)
+    keys = rng.integers(0, d, n).astype(dtype)
+    keys[7::1000], keys[8::999] = info.min, info.max
+    if dtype == np.uint64:
+        keys[9::501] = 1 << 63
+    vals = rng.integers(-1000, 1000, n).astype(np.int64)
+    f = rng.random(n).astype(np.float32)
+    for reqs in ([(0, A.SUM), (-1, A.COUNT_ALL)], [(0, A.MIN), (0, A.MAX), (1, A.SUM), (-1, A.COUNT_ALL), (0, A.SUM)]):
+        exp = sorted_by_key(O.groupby(keys, [vals, f], reqs))
+        for bound in (len(exp[0]), max(1, len(exp[0]) // 3)):
+            got = sorted_by_key(run(G.hash_groupby, keys, [vals, f], reqs, G.groupby_hint(groups_upper_bound=bound)))
+            assert_same(got, exp)
