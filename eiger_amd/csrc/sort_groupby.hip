@@ -12,7 +12,7 @@
 //      (SORT_GFUR: values are gathered through the permutation, like the
 //      reference's permutation_iterator, groupby_sort.cu:429-479);
 //   3. a segmented reduction that computes every aggregation in one pass:
-//      seg_heads_kernel counts group heads per 4096-row tile, a scan gives each
+//      seg_heads_kernel counts group heads per tile, a scan gives each
 //      tile its first group index, and seg_reduce_kernel folds each lane's
 //      consecutive rows in registers, merges runs that cross lanes through LDS
 //      states, writes the tile's complete groups and hands the group that
@@ -140,7 +140,10 @@ __device__ __forceinline__ void emit_regs(const OutSpec& os, int64_t g, uint64_t
     }
 }
 
-// One 4096-row tile of sorted rows (ITEMS consecutive rows per lane).  A run
+// One tile of sorted rows (ITEMS consecutive rows per lane).  Each column is
+// read lane by lane and turned through LDS (a lane reading its own
+// consecutive rows makes every load 64 cache lines: 40M rows of int64 keys and
+// double values took 583 us).  A run
 // (rows of one key) that starts and ends inside a lane is folded in registers
 // and written straight out.  Runs that cross lane boundaries meet in LDS:
 // slot L (nops states) collects the group whose head is in lane L, slot
@@ -162,6 +165,7 @@ __global__ __launch_bounds__(kSegB) void seg_reduce_kernel(const void* keys, int
     constexpr int kb = KB;
     (void)kb_unused;
     extern __shared__ unsigned long long slot[];  // nops * kSlots
+    __shared__ unsigned long long turn[kSegB * (ITEMS + 1)];  // a column of the tile, one word of padding per lane
     __shared__ uint32_t wsum[kSegB / 64];
     __shared__ int wmax[kSegB / 64];
     __shared__ uint32_t s_tile_cont;
@@ -180,9 +184,21 @@ __global__ __launch_bounds__(kSegB) void seg_reduce_kernel(const void* keys, int
     auto key_at = [&](int64_t r) -> uint64_t {
         return KB == 4 ? (uint64_t)((const uint32_t*)keys)[r] : ((const uint64_t*)keys)[r];
     };
+    // load(r) for every row of the tile, into this lane's consecutive rows
+    auto turned = [&](auto load, uint64_t (&o)[ITEMS]) {
 #pragma unroll
-    for (int i = 0; i < ITEMS; ++i) k[i] = r0 + i < n ? key_at(r0 + i) : 0ull;
-    uint64_t prev = (r0 > 0 && r0 < n) ? key_at(r0 - 1) : 0ull;
+        for (int i = 0; i < ITEMS; ++i) {
+            const int e = i * kSegB + t;
+            const int64_t r = tstart + e;
+            turn[e + e / ITEMS] = r < n ? load(r) : 0ull;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) o[i] = turn[t * (ITEMS + 1) + i];
+    };
+    turned(key_at, k);
+    uint64_t prev = 0ull;
+    if (r0 > 0 && r0 < n) prev = t > 0 ? turn[(t - 1) * (ITEMS + 1) + ITEMS - 1] : key_at(r0 - 1);
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
         const int64_t r = r0 + i;
@@ -191,7 +207,9 @@ __global__ __launch_bounds__(kSegB) void seg_reduce_kernel(const void* keys, int
         prev = k[i];
     }
     const int64_t r_end = r0 + ITEMS;  // first row after this lane
-    const bool next_head = r_end >= n || (r0 < n && key_at(r_end) != k[ITEMS - 1]);
+    bool next_head = r_end >= n;
+    if (!next_head) next_head = (t + 1 < kSegB ? turn[(t + 1) * (ITEMS + 1)] : key_at(r_end)) != k[ITEMS - 1];
+    __syncthreads();  // turn is free again
     // groups whose head precedes this lane within the tile, and the tile total
     uint32_t tile_heads = 0;
     const uint32_t hbefore = block_excl_scan(nheads, wsum, &tile_heads);
@@ -241,24 +259,26 @@ __global__ __launch_bounds__(kSegB) void seg_reduce_kernel(const void* keys, int
             to_slot(t);
         }
     };
-    // values of the lane's rows: typed loads issued eight rows at a time
-    // (fixed layouts), then folded
-    constexpr int H = 8;
-    static_assert(ITEMS % H == 0, "rows per lane in halves");
-#pragma unroll
-    for (int h0 = 0; h0 < ITEMS; h0 += H) {
-    uint64_t rawv[VL::GEN ? 1 : H][NV];
-    if constexpr (!VL::GEN) {
-#pragma unroll
-        for (int j = 0; j < H; ++j) {
-            const int64_t r = r0 + h0 + j;
-            const bool valid = r < n;
-            load_row<VL>(spec, valid ? (perm ? perm[r] : r) : 0, valid, rawv[j]);
+    // values of the lane's rows (wide layouts: typed loads row by row)
+    uint64_t rawv[VL::GEN ? 1 : NV][ITEMS];
+    if constexpr (!VL::GEN && VL::NV >= 1) {
+        auto column = [&](auto c) {
+            constexpr int C = decltype(c)::value;
+            constexpr int W = VL::template width<C>();
+            const void* data = spec.cols[C].data;
+            turned([&](int64_t r) -> uint64_t {
+                const int64_t x = perm ? perm[r] : r;
+                return W == 4 ? (uint64_t)((const uint32_t*)data)[x] : ((const uint64_t*)data)[x];
+            }, rawv[C]);
+        };
+        column(std::integral_constant<int, 0>{});
+        if constexpr (VL::NV >= 2) {
+            __syncthreads();
+            column(std::integral_constant<int, 1>{});
         }
     }
 #pragma unroll
-    for (int j = 0; j < H; ++j) {
-        const int i = h0 + j;
+    for (int i = 0; i < ITEMS; ++i) {
         const int64_t r = r0 + i;
         if (r >= n) break;
         if (head[i]) {
@@ -268,14 +288,14 @@ __global__ __launch_bounds__(kSegB) void seg_reduce_kernel(const void* keys, int
             ++hseen;
             run_key = k[i];
         }
-        uint64_t cv[NV];
+        uint64_t cv[NV], raw[NV];
         if constexpr (VL::GEN) {
-            uint64_t raw[NV];
             load_row<VL>(spec, perm ? perm[r] : r, true, raw);
-            canon_row<VL, NV>(spec, raw, cv);
         } else {
-            canon_row<VL, NV>(spec, rawv[j], cv);
+#pragma unroll
+            for (int c = 0; c < NV; ++c) raw[c] = VL::NV > 0 ? rawv[c][i] : 0ull;
         }
+        canon_row<VL, NV>(spec, raw, cv);
 #pragma unroll
         for (int a = 0; a < kMaxOps; ++a) {
             if (a < nops) {
@@ -289,7 +309,6 @@ __global__ __launch_bounds__(kSegB) void seg_reduce_kernel(const void* keys, int
             }
         }
         have = true;
-    }
     }
     // the lane's last run: complete when the next row starts a new group
     finish(next_head);
@@ -361,7 +380,7 @@ Result reduce_sorted(const Plan& plan, const void* sorted_keys, const AggSpec& s
 {
     const int64_t n = plan.rows;
     const int kb = plan.key.bytes;
-    constexpr int items = 16;
+    constexpr int items = 8;  // 2048-row tiles: the turned column and five states leave five workgroups a CU
     const int T = kSegB * items;
     const int64_t ntiles64 = (n + T - 1) / T;
     if (ntiles64 >= ((int64_t)1 << 31)) raise(EG_ERR_UNSUPPORTED, "too many rows for the segmented reduction");
