@@ -111,11 +111,13 @@ __device__ __forceinline__ void gt_count_inserts(const GTable& gt, uint32_t ins)
 #ifndef __HIPCC_RTC__  // host side
 int table_words_per_slot(int nops);
 
-// Owns a zeroed HBM table of `slots` (power of two) slots.
+// Owns a zeroed HBM table of `slots` (power of two) slots; `extra` zeroed
+// words follow its four meta words (at meta + 4).
 struct HbmTable {
     DevBuf buf;
     GTable gt;
-    HbmTable(int64_t slots, int W, hipStream_t s);
+    unsigned long long* extra = nullptr;
+    HbmTable(int64_t slots, int W, hipStream_t s, int64_t extra_words = 0);
     void read_meta(int64_t* out3, hipStream_t s);   // synchronises s
     // Appends every occupied slot to the outputs at positions from *counter.
     void compact(const OutSpec& os, unsigned long long* counter, hipStream_t s);

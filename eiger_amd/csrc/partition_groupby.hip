@@ -150,6 +150,67 @@ __global__ __launch_bounds__(256) void units_fill_kernel(const int64_t* __restri
     if (p == P - 1) meta[1] = (unsigned long long)pre[p] + k;
 }
 
+// Boundaries and units of up to kUnitsSmall partitions in one launch of one
+// workgroup (five launches otherwise): thread t finds the first rows of its
+// consecutive partitions by binary search, then one scan places the units.
+constexpr int kUnitsPer = 4;
+constexpr int64_t kUnitsSmall = 1024 * kUnitsPer;
+
+template <int KB>
+__global__ __launch_bounds__(1024) void units_small_kernel(const void* __restrict__ keys, int64_t n, uint32_t mask,
+                                                           int64_t P, int64_t slice, agg::Unit* __restrict__ units,
+                                                           unsigned long long* meta)
+{
+    __shared__ uint32_t wsum[16];
+    __shared__ int64_t first[1024 * kUnitsPer + 1];
+    __shared__ uint32_t s_sliced;
+    const int t = threadIdx.x;
+    const int per = (int)((P + 1023) / 1024);
+    if (t == 0) s_sliced = 0u;
+    int64_t lo[kUnitsPer], hi[kUnitsPer];
+#pragma unroll
+    for (int i = 0; i < kUnitsPer; ++i) lo[i] = 0, hi[i] = i < per && (int64_t)t * per + i < P ? n : 0;
+    bool more = true;
+    while (more) {  // rows < lo have id < p, rows >= hi have id >= p; the searches side by side
+        more = false;
+#pragma unroll
+        for (int i = 0; i < kUnitsPer; ++i) {
+            if (lo[i] >= hi[i]) continue;
+            const int64_t mid = lo[i] + ((hi[i] - lo[i]) >> 1);
+            if ((int64_t)pid_of<KB>(dev::load_raw(keys, KB, mid), mask) < (int64_t)t * per + i) lo[i] = mid + 1;
+            else hi[i] = mid;
+            more = more || lo[i] < hi[i];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kUnitsPer; ++i)
+        if (i < per && (int64_t)t * per + i < P) first[t * per + i] = lo[i];
+    if (t == 0) first[P] = n;
+    __syncthreads();
+    uint32_t cnt[kUnitsPer], sum = 0, sliced = 0;
+#pragma unroll
+    for (int i = 0; i < kUnitsPer; ++i) {
+        cnt[i] = 0;
+        if (i < per && (int64_t)t * per + i < P) {
+            const int64_t rows = first[t * per + i + 1] - first[t * per + i];
+            cnt[i] = rows <= 0 ? 0u : rows <= slice ? 1u : (uint32_t)((rows + slice - 1) / slice);
+            sliced += rows > slice ? 1u : 0u;
+        }
+        sum += cnt[i];
+    }
+    if (sliced) atomicAdd(&s_sliced, sliced);
+    uint32_t at = dev::block_excl_scan<1024>(sum, wsum);
+    if (t == 1023) meta[1] = (unsigned long long)at + sum;
+#pragma unroll
+    for (int i = 0; i < kUnitsPer; ++i)
+        for (uint32_t j = 0; j < cnt[i]; ++j) {
+            const int64_t x = first[t * per + i] + (int64_t)j * slice, e = first[t * per + i + 1];
+            units[at++] = agg::Unit{x, cnt[i] == 1 ? e : (x + slice < e ? x + slice : e), cnt[i] > 1 ? 1 : 0, 0};
+        }
+    __syncthreads();
+    if (t == 0) meta[0] = s_sliced;
+}
+
 // Output rows past the group count moved into the holes below it (the
 // unused tails of the lanes' last chunks): op i copies len[i] rows from
 // src[i] to dst[i] in every output column; sources and destinations are
@@ -215,8 +276,13 @@ Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream
     while (cr > 64 && lds_of(cr) + static_lds > (size_t)di.max_lds) cr -= 4;
     const size_t lds = lds_of(cr);
     const int64_t per_part = std::max<int64_t>(1, (int64_t)cr * 2 / 3);  // target groups per partition
-    const int bits = std::min(24, std::max(1, ceil_log2((bound + per_part - 1) / per_part)));
+    int bits = std::min(24, std::max(1, ceil_log2((bound + per_part - 1) / per_part)));
     const int digit_bits = max_digit_bits();
+    // Fewer radix passes where the tables then fill to 7/8 of the bound at
+    // most (the bound is an upper one, and an estimate's carries headroom):
+    // 3M rows with a bound of 600k groups take one 8-bit pass instead of two.
+    const int fewer = (bits + digit_bits - 1) / digit_bits * digit_bits - digit_bits;
+    if (fewer >= digit_bits && (bound >> fewer) <= (int64_t)cr * 7 / 8) bits = fewer;
     const uint32_t pmask = (uint32_t)((1u << bits) - 1u);
 
     std::unique_ptr<HostPhase> phase_prep(new HostPhase("host_partition_prep", s));
@@ -291,14 +357,6 @@ Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream
     // ---- partition boundaries and units -------------------------------------------
     const int64_t P = (int64_t)pmask + 1;
     std::unique_ptr<HostPhase> phase_units(new HostPhase("host_partition_units", s));
-    DevBuf offs((size_t)(P + 1) * 8, s);
-    {
-        const int64_t grid = (P + 1 + 255) / 256;  // one thread per boundary
-        KernelTimer timer("partition_bounds", s);
-        if (kb == 4) hipLaunchKernelGGL(part_bounds_kernel<4>, dim3((unsigned)grid), dim3(256), 0, s, pkeys, n, pmask, offs.get<int64_t>());
-        else hipLaunchKernelGGL(part_bounds_kernel<8>, dim3((unsigned)grid), dim3(256), 0, s, pkeys, n, pmask, offs.get<int64_t>());
-        EG_LAUNCH_CHECK();
-    }
     // Rows per unit: a partition is split when it is much larger than the
     // average (skew), or when there are too few partitions to occupy every CU
     // twice, since a split partition's groups merge through the HBM table with
@@ -320,15 +378,31 @@ Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream
         uint32_t* cnt = ub.get<uint32_t>();
         uint32_t* pre = cnt + P;
         unsigned long long* umeta = reinterpret_cast<unsigned long long*>(pre + P);
-        EG_HIP(hipMemsetAsync(umeta, 0, 16, s));
-        const unsigned ugrid = (unsigned)((P + 255) / 256);
-        hipLaunchKernelGGL(units_count_kernel, dim3(ugrid), dim3(256), 0, s, (const int64_t*)offs.get<int64_t>(), P,
-                           slice, cnt, umeta);
-        EG_LAUNCH_CHECK();
-        scan_exclusive_u32(cnt, pre, P, s, false);
-        hipLaunchKernelGGL(units_fill_kernel, dim3(ugrid), dim3(256), 0, s, (const int64_t*)offs.get<int64_t>(), P,
-                           slice, (const uint32_t*)cnt, (const uint32_t*)pre, dunits.get<Unit>(), umeta);
-        EG_LAUNCH_CHECK();
+        DevBuf offs;
+        if (P <= kUnitsSmall) {
+            KernelTimer timer("partition_bounds", s);
+            auto kern = kb == 4 ? units_small_kernel<4> : units_small_kernel<8>;
+            hipLaunchKernelGGL(kern, dim3(1), dim3(1024), 0, s, pkeys, n, pmask, P, slice, dunits.get<Unit>(), umeta);
+            EG_LAUNCH_CHECK();
+        } else {
+            offs = DevBuf((size_t)(P + 1) * 8, s);
+            {
+                const int64_t grid = (P + 1 + 255) / 256;  // one thread per boundary
+                KernelTimer timer("partition_bounds", s);
+                if (kb == 4) hipLaunchKernelGGL(part_bounds_kernel<4>, dim3((unsigned)grid), dim3(256), 0, s, pkeys, n, pmask, offs.get<int64_t>());
+                else hipLaunchKernelGGL(part_bounds_kernel<8>, dim3((unsigned)grid), dim3(256), 0, s, pkeys, n, pmask, offs.get<int64_t>());
+                EG_LAUNCH_CHECK();
+            }
+            fill_zero(umeta, 16, s);
+            const unsigned ugrid = (unsigned)((P + 255) / 256);
+            hipLaunchKernelGGL(units_count_kernel, dim3(ugrid), dim3(256), 0, s, (const int64_t*)offs.get<int64_t>(), P,
+                               slice, cnt, umeta);
+            EG_LAUNCH_CHECK();
+            scan_exclusive_u32(cnt, pre, P, s, false);
+            hipLaunchKernelGGL(units_fill_kernel, dim3(ugrid), dim3(256), 0, s, (const int64_t*)offs.get<int64_t>(), P,
+                               slice, (const uint32_t*)cnt, (const uint32_t*)pre, dunits.get<Unit>(), umeta);
+            EG_LAUNCH_CHECK();
+        }
         int64_t* hm = pinned_i64(2);
         EG_HIP(hipMemcpyAsync(hm, umeta, 16, hipMemcpyDeviceToHost, s));
         EG_HIP(hipStreamSynchronize(s));
@@ -359,14 +433,12 @@ Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream
         Result res;
         OutSpec os;
         alloc_outputs(plan, cap_rows, s, res, os);
-        HbmTable ht(slots, W, s);
         OutClaims claims;
         claims.chunk = chunk;
         claims.maxc = cap_rows / chunk + 2;
-        const size_t claim_bytes = (size_t)agg::claim_words(claims.maxc) * 8;
-        DevBuf cbuf(claim_bytes, s);
-        fill_zero(cbuf.get(), claim_bytes, s);
-        claims.words = cbuf.get<unsigned long long>();
+        // the claims follow the table's meta words: one fill, one read back
+        HbmTable ht(slots, W, s, agg::claim_words(claims.maxc));
+        claims.words = ht.extra;
         if (kb == 4)
             launch_part<4>(gfur, pkey, spec, perm, dunits.get<Unit>(), (int)nunits, ht.gt, os, claims,
                            cap_rows, cr, lds, tune.block, n, s);
@@ -386,10 +458,9 @@ Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream
             EG_LAUNCH_CHECK();
         }
         // the claims' head and the table's meta words in one synchronisation
-        int64_t* h = (int64_t*)pinned_staging((size_t)agg::kClaimHeadWords * 8, 2);
-        int64_t* hm = pinned_i64(4);
-        EG_HIP(hipMemcpyAsync(h, claims.words, (size_t)agg::kClaimHeadWords * 8, hipMemcpyDeviceToHost, s));
-        EG_HIP(hipMemcpyAsync(hm, ht.gt.meta, 3 * sizeof(int64_t), hipMemcpyDeviceToHost, s));
+        int64_t* hm = (int64_t*)pinned_staging((size_t)(4 + agg::kClaimHeadWords) * 8, 2);
+        const int64_t* h = hm + 4;
+        EG_HIP(hipMemcpyAsync(hm, ht.gt.meta, (size_t)(4 + agg::kClaimHeadWords) * 8, hipMemcpyDeviceToHost, s));
         EG_HIP(hipStreamSynchronize(s));
         const int64_t meta[3] = {hm[0], hm[1], hm[2]};
         const bool table_full = meta[2] != 0;

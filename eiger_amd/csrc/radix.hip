@@ -330,6 +330,38 @@ __global__ __launch_bounds__(kOB) void tile_offsets_kernel(const uint32_t* __res
     }
 }
 
+// Small passes: the same offsets in one launch of one workgroup (the three
+// launches cost more than the counts).  Threads form 1024 / nd segments of
+// consecutive tiles per digit: sums per segment, a scan over segments and
+// digits, then the walk.
+constexpr int kSmallCounts = 1 << 16;  // counts up to which one workgroup does it
+
+__global__ __launch_bounds__(1024) void tile_offsets_small_kernel(const uint32_t* __restrict__ counts, int ntiles,
+                                                                  int nd, uint32_t* __restrict__ offs)
+{
+    __shared__ uint32_t wsum[16];
+    __shared__ uint32_t seg[1024];
+    const int d = threadIdx.x % nd, g = threadIdx.x / nd, ns = 1024 / nd;  // nd: a power of two <= 256
+    const int per = (ntiles + ns - 1) / ns;
+    const int t0 = min(ntiles, g * per), t1 = min(ntiles, t0 + per);
+    uint32_t sum = 0;
+#pragma unroll 8
+    for (int t = t0; t < t1; ++t) sum += counts[(int64_t)t * nd + d];
+    seg[d * ns + g] = sum;  // digit-major: the scan below is over (digit, segment)
+    __syncthreads();
+    const uint32_t ex = block_excl_scan<1024>(seg[threadIdx.x], wsum);
+    __syncthreads();
+    seg[threadIdx.x] = ex;
+    __syncthreads();
+    uint32_t run = seg[d * ns + g];
+#pragma unroll 8
+    for (int t = t0; t < t1; ++t) {
+        const uint32_t c = counts[(int64_t)t * nd + d];
+        offs[(int64_t)t * nd + d] = run;
+        run += c;
+    }
+}
+
 // ---- device-wide exclusive scan of uint32 (reduce, scan the block sums, add) ----
 constexpr int kSB = 256, kSI = 16, kST = kSB * kSI;
 
@@ -527,6 +559,11 @@ void radix_pass(const RadixKeys& k, void* keys_out, const std::vector<Payload>& 
     }
     {
         KernelTimer timer("radix_scan", s);
+        if (nh <= kSmallCounts) {
+            hipLaunchKernelGGL(tile_offsets_small_kernel, dim3(1), dim3(1024), 0, s, (const uint32_t*)hist.get<uint32_t>(),
+                               ntiles, nd, offs.get<uint32_t>());
+            EG_LAUNCH_CHECK();
+        } else {
         const int per = std::max(16, (ntiles + 4095) / 4096);  // tiles per chunk: at most 4096 chunks
         const int nchunks = (ntiles + per - 1) / per;
         DevBuf cs((size_t)nchunks * nd * 4 * 2 + (size_t)nd * 4, s);
@@ -542,6 +579,7 @@ void radix_pass(const RadixKeys& k, void* keys_out, const std::vector<Payload>& 
         hipLaunchKernelGGL(tile_offsets_kernel, dim3(nchunks), dim3(kOB), 0, s, (const uint32_t*)hist.get<uint32_t>(),
                            ntiles, nd, per, (const uint32_t*)coff, (const uint32_t*)total, offs.get<uint32_t>());
         EG_LAUNCH_CHECK();
+        }
     }
     PayArgs pa{};
     pa.n = (int32_t)pay.size();
