@@ -25,6 +25,7 @@ void timing_query(const char* name, int64_t* launches, double* total_ms);
 void zipf_cdf(double* cdf, int64_t distinct, double s);
 Result run_sort(const Plan& plan, const eg_groupby_hint& hint, bool gfur, hipStream_t s);
 Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream_t s);
+int partition_passes(const Plan& plan, int64_t group_bound);  // its radix passes at this bound
 bool mlp_select(const void* keys, int32_t key_type, int64_t rows, int64_t group_bound, int nops, int value_bytes,
                 hipStream_t s, int32_t* algo, int64_t* card_est, float* singletons);
 int64_t ndv_approx(const void* data, int32_t type, int64_t n, hipStream_t s);
@@ -430,15 +431,27 @@ int groupby_entry(Entry entry, const eg_column_view* keys, int64_t num_keys,
                     // (more than 1/4 of its keys seen once) the full-column
                     // HyperLogLog estimate (standard error 0.8%, 25% headroom)
                     // sizes the tables instead: one pass over the keys, cheap
-                    // against such an input, and tighter tables.  Below that
-                    // the pass and its synchronisation would cost more than
-                    // the tighter sizing saves; the model's estimate stays
-                    // within 1.34x of the true count on every held-out query
-                    // of that kind (2,913), far inside the headroom.
-                    const int64_t caller = (h.groups_upper_bound > 0 && h.groups_upper_bound < plan.rows)
-                                               ? h.groups_upper_bound : plan.rows;
+                    // against such an input, and tighter tables.  With no
+                    // caller bound it runs whatever the estimate (67M rows in
+                    // 16.7M groups were cut into 32768 partitions for the row
+                    // count as bound: 2.98 -> 2.75 ms).  With one, and the
+                    // partition strategy, only where a tighter bound could
+                    // save a radix pass or two digit bits of two passes: else
+                    // it costs more (0.25 ms per 2^28 rows) than it saves.
+                    // Below 2^24 rows the pass and its synchronisation would
+                    // cost more than the tighter sizing saves; the model's
+                    // estimate stays within 1.34x of the true count on every
+                    // held-out query of that kind (2,913), far inside the
+                    // headroom.
+                    const bool known = h.groups_upper_bound > 0 && h.groups_upper_bound < plan.rows;
+                    const int64_t caller = known ? h.groups_upper_bound : plan.rows;
                     learned_bound = std::min<int64_t>(caller, card + card + card / 2 + 1024);
-                    if (learned_bound < caller && singletons > 0.25f && plan.rows >= ((int64_t)1 << 24)) {
+                    const int passes = known && a == EG_ALGO_PARTITION ? partition_passes(plan, caller) : 0;
+                    if (plan.rows >= ((int64_t)1 << 24) && passes > 0 && passes == partition_passes(plan, learned_bound) &&
+                        (passes == 1 || 4 * learned_bound >= caller)) {
+                        learned_bound = caller;
+                    } else if ((learned_bound < caller || !known) && singletons > 0.25f &&
+                               plan.rows >= ((int64_t)1 << 24)) {
                         const int64_t est = ndv_approx(plan.key.data, plan.key_type, plan.rows, s);
                         learned_bound = std::min<int64_t>(caller, est + est / 4 + 1024);
                     }

@@ -114,6 +114,7 @@ __global__ __launch_bounds__(256) void part_compact_kernel(GTable gt, OutSpec os
                                                            int64_t capacity)
 {
     __shared__ unsigned long long sh[17];
+    if (gt.meta[0] == 0ull && gt.meta[1] == 0ull) return;  // nothing spilled and no partition was sliced
     compact_groups<kCompactSlots>(gt, counter, sh, [&](int64_t idx, uint64_t enc, const unsigned long long* st) {
         if (idx < capacity) dev::emit_group(os, idx, enc, st, 1);
     });
@@ -153,8 +154,10 @@ __global__ __launch_bounds__(256) void units_fill_kernel(const int64_t* __restri
 // Boundaries and units of up to kUnitsSmall partitions in one launch of one
 // workgroup (five launches otherwise): thread t finds the first rows of its
 // consecutive partitions by binary search, then one scan places the units.
-constexpr int kUnitsPer = 4;
-constexpr int64_t kUnitsSmall = 1024 * kUnitsPer;
+// Above, one CU's searches take longer than the launches (4096 partitions of
+// 2^28 rows: 168 us against ~35).
+constexpr int kUnitsPer = 1;
+constexpr int64_t kUnitsSmall = 512;
 
 template <int KB>
 __global__ __launch_bounds__(1024) void units_small_kernel(const void* __restrict__ keys, int64_t n, uint32_t mask,
@@ -162,7 +165,7 @@ __global__ __launch_bounds__(1024) void units_small_kernel(const void* __restric
                                                            unsigned long long* meta)
 {
     __shared__ uint32_t wsum[16];
-    __shared__ int64_t first[1024 * kUnitsPer + 1];
+    __shared__ int64_t first[kUnitsSmall + 1];
     __shared__ uint32_t s_sliced;
     const int t = threadIdx.x;
     const int per = (int)((P + 1023) / 1024);
@@ -252,7 +255,49 @@ void launch_part(bool gather, const KeyDesc& key, const AggSpec& spec, const int
                                    rows, s);
 }
 
+// LDS table and workgroup (see PartTune), and the partition count: chosen so
+// a partition holds about 2/3 of the table.
+struct PartGeometry {
+    PartTune tune;
+    int cr;
+    size_t lds;
+    int64_t per_part;  // target groups per partition
+    int bits;          // log2 partitions
+};
+
+PartGeometry part_geometry(int nops, int kb, int64_t bound)
+{
+    const DeviceInfo& di = device_info();
+    PartGeometry g;
+    g.tune = part_tune();
+    const size_t static_lds = 256;
+    auto lds_of = [&](int c) { return (size_t)agg::unit_table_words(nops, c, kb) * 8; };
+    g.cr = g.tune.cr;
+    if (g.cr == 0) {
+        const size_t budget = std::min<size_t>((size_t)di.max_lds, 160 * 1024) / 2 - static_lds;
+        g.cr = 4;
+        while (g.cr < 16384 && lds_of(g.cr + 4) <= budget) g.cr += 4;
+    }
+    while (g.cr > 64 && lds_of(g.cr) + static_lds > (size_t)di.max_lds) g.cr -= 4;
+    g.lds = lds_of(g.cr);
+    g.per_part = std::max<int64_t>(1, (int64_t)g.cr * 2 / 3);
+    g.bits = std::min(24, std::max(1, ceil_log2((bound + g.per_part - 1) / g.per_part)));
+    // Fewer radix passes where the tables then fill to 7/8 of the bound at
+    // most (the bound is an upper one, and an estimate's carries headroom):
+    // 3M rows with a bound of 600k groups take one 8-bit pass instead of two.
+    const int digit_bits = max_digit_bits();
+    const int fewer = (g.bits + digit_bits - 1) / digit_bits * digit_bits - digit_bits;
+    if (fewer >= digit_bits && (bound >> fewer) <= (int64_t)g.cr * 7 / 8) g.bits = fewer;
+    return g;
+}
+
 }  // namespace
+
+int partition_passes(const Plan& plan, int64_t group_bound)
+{
+    const int64_t bound = std::max<int64_t>(1, std::min<int64_t>(group_bound, plan.rows));
+    return (part_geometry(plan.spec.nops, plan.key.bytes, bound).bits + max_digit_bits() - 1) / max_digit_bits();
+}
 
 Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream_t s)
 {
@@ -262,27 +307,12 @@ Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream
     const int nops = plan.spec.nops;
     const int64_t bound = std::max<int64_t>(1, std::min<int64_t>(group_bound, n));
 
-    // LDS table and workgroup (see PartTune); the partition count is chosen
-    // so a partition holds about 2/3 of the table.
-    const PartTune tune = part_tune();
-    const size_t static_lds = 256;
-    auto lds_of = [&](int c) { return (size_t)agg::unit_table_words(nops, c, kb) * 8; };
-    int cr = tune.cr;
-    if (cr == 0) {
-        const size_t budget = std::min<size_t>((size_t)di.max_lds, 160 * 1024) / 2 - static_lds;
-        cr = 4;
-        while (cr < 16384 && lds_of(cr + 4) <= budget) cr += 4;
-    }
-    while (cr > 64 && lds_of(cr) + static_lds > (size_t)di.max_lds) cr -= 4;
-    const size_t lds = lds_of(cr);
-    const int64_t per_part = std::max<int64_t>(1, (int64_t)cr * 2 / 3);  // target groups per partition
-    int bits = std::min(24, std::max(1, ceil_log2((bound + per_part - 1) / per_part)));
+    const PartGeometry geo = part_geometry(nops, kb, bound);
+    const PartTune tune = geo.tune;
+    const int cr = geo.cr, bits = geo.bits;
+    const size_t lds = geo.lds;
+    const int64_t per_part = geo.per_part;
     const int digit_bits = max_digit_bits();
-    // Fewer radix passes where the tables then fill to 7/8 of the bound at
-    // most (the bound is an upper one, and an estimate's carries headroom):
-    // 3M rows with a bound of 600k groups take one 8-bit pass instead of two.
-    const int fewer = (bits + digit_bits - 1) / digit_bits * digit_bits - digit_bits;
-    if (fewer >= digit_bits && (bound >> fewer) <= (int64_t)cr * 7 / 8) bits = fewer;
     const uint32_t pmask = (uint32_t)((1u << bits) - 1u);
 
     std::unique_ptr<HostPhase> phase_prep(new HostPhase("host_partition_prep", s));
