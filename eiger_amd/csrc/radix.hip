@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "eg_device.hpp"
 #include "eg_internal.hpp"
@@ -137,16 +138,26 @@ __device__ __forceinline__ void stage_column(const uint64_t (&v)[kRI], const uin
         if (pos[i] != 0xffffffffu) stage[pos[i]] = v[i];
 }
 
+// Rows of a cache line that lies whole inside the run are stored
+// non-temporally: nothing else will touch that line, while the run's ragged
+// end lines wait in the L2 for the neighbouring tile's rows.
 template <int B>
 __device__ __forceinline__ void store_column_w(void* dst, int t, int32_t tcount, const unsigned long long* stage,
                                                const uint8_t* sdig, const uint32_t* gofs, const uint32_t* lstart)
 {
+    using T = typename std::conditional<B == 1, uint8_t, typename std::conditional<B == 2, uint16_t,
+              typename std::conditional<B == 4, uint32_t, unsigned long long>::type>::type>::type;
+    constexpr uint32_t kLine = 128 / B;  // elements; the output columns start on a line
 #pragma unroll
     for (int i = 0; i < kRI; ++i) {
         const int p = i * kRB + t;
         if (p < tcount) {
             const uint32_t d = sdig[p];
-            store_key<B>(dst, (int64_t)gofs[d] + (p - (int64_t)lstart[d]), stage[p]);
+            const uint32_t g = gofs[d], l = lstart[d], to = g + ((uint32_t)p - l);
+            const uint32_t last = g + (lstart[d + 1] - l - 1u);  // the run's last row
+            T* at = (T*)dst + to;
+            if ((to & ~(kLine - 1u)) >= g && (to | (kLine - 1u)) <= last) __builtin_nontemporal_store((T)stage[p], at);
+            else *at = (T)stage[p];
         }
     }
 }
@@ -180,7 +191,7 @@ __global__ __launch_bounds__(kRB) void radix_scatter_kernel(RadixKeys k, void* _
     __shared__ unsigned long long stage[kRT];
     __shared__ uint8_t sdig[kRT];
     __shared__ uint32_t whist[kW][256];
-    __shared__ uint32_t lstart[256];
+    __shared__ uint32_t lstart[257];
     __shared__ uint32_t gofs[256];
     __shared__ uint32_t wsum[kW];
 
@@ -239,6 +250,7 @@ __global__ __launch_bounds__(kRB) void radix_scatter_kernel(RadixKeys k, void* _
     }
     const uint32_t ls = block_excl_scan256(run, wsum);
     lstart[t] = ls;
+    if (t == kRB - 1) lstart[256] = ls + run;
     __syncthreads();
     const int32_t tcount = (int32_t)min<int64_t>((int64_t)kRT, n - tbase);
     uint32_t pos[kRI];
