@@ -1,5 +1,5 @@
 // eg_seg_launch.hpp -- launch of the segmented reduction: one translation unit
-// instantiates it per key width (seg_reduce*.hip).
+// instantiates it per key width and number of states (seg_reduce*.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -13,6 +13,11 @@ constexpr int kSegB = 256;
 // 2048-row tiles: the turned column and five states leave five workgroups a CU.
 constexpr int kSegItems = 8;
 
+// Requests of at most this many states take kernels unrolled for that many,
+// half the code and 67 instead of 88 registers (40M rows of int64 keys and
+// doubles, three states: 1.64 against 1.75 ms a call); others kMaxOps.
+constexpr int kSegFewOps = 6;
+
 struct SegArgs {
     const void* keys;
     const int64_t* perm;
@@ -24,7 +29,7 @@ struct SegArgs {
     uint32_t* btrail;
 };
 
-template <int KB>
+template <int KB, int MO>
 void launch_seg(const SegArgs& a, int is_signed, const AggSpec& spec, const OutSpec& os, hipStream_t s);
 
 }  // namespace eg

@@ -47,14 +47,15 @@ __device__ __forceinline__ uint32_t owner_tile(const uint32_t* head_off, uint32_
 }
 
 // Writes group g from states held in registers.
-__device__ __forceinline__ void emit_regs(const OutSpec& os, int64_t g, uint64_t key_enc, const uint64_t (&acc)[kMaxOps])
+template <int MO>
+__device__ __forceinline__ void emit_regs(const OutSpec& os, int64_t g, uint64_t key_enc, const uint64_t (&acc)[MO])
 {
     dev::store_bytes(os.key_data, os.key_bytes, g, dev::dec64(key_enc));
     for (int j = 0; j < os.nouts; ++j) {
         const OutDesc& o = os.outs[j];
         uint64_t st[2] = {0ull, 0ull};
 #pragma unroll
-        for (int a = 0; a < kMaxOps; ++a) {
+        for (int a = 0; a < MO; ++a) {
             if (a == o.op) st[0] = acc[a];
             if (a == o.op2) st[1] = acc[a];
         }
@@ -97,7 +98,7 @@ __device__ __forceinline__ void emit_regs(const OutSpec& os, int64_t g, uint64_t
 // group, if it continues into the next tile, goes to the tile's boundary
 // state instead; the continuation group of an earlier tile's head is added
 // to that tile's boundary state.
-template <int KB, class VL>
+template <int KB, int MO, class VL>
 __global__ __launch_bounds__(kSegB) void seg_reduce_kernel(SegArgs sa, int is_signed, AggSpec spec, OutSpec os)
 {
     constexpr int ITEMS = kSegItems;
@@ -185,15 +186,15 @@ __global__ __launch_bounds__(kSegB) void seg_reduce_kernel(SegArgs sa, int is_si
         return nx < n && key_at(nx) == key_at(nx - 1);
     }();
 
-    uint64_t acc[kMaxOps];
+    uint64_t acc[MO];
 #pragma unroll
-    for (int a = 0; a < kMaxOps; ++a) acc[a] = 0ull;
+    for (int a = 0; a < MO; ++a) acc[a] = 0ull;
     bool have = false, cont = r0 < n && r0 > 0 && !head[0];
     uint32_t hseen = 0;          // heads of this lane seen so far
     uint64_t run_key = 0;
     auto to_slot = [&](int sidx) {
 #pragma unroll
-        for (int a = 0; a < kMaxOps; ++a)
+        for (int a = 0; a < MO; ++a)
             if (a < nops) dev::apply_atomic(dev::class_of(spec, a), &slot[(size_t)a * kSlots + sidx], acc[a]);
     };
     // closes the current run; `closed`: the run ends inside this lane
@@ -246,7 +247,7 @@ __global__ __launch_bounds__(kSegB) void seg_reduce_kernel(SegArgs sa, int is_si
         }
         canon_row<VL, NV>(spec, raw, cv);
 #pragma unroll
-        for (int a = 0; a < kMaxOps; ++a) {
+        for (int a = 0; a < MO; ++a) {
             if (a < nops) {
                 const OpDesc od = spec.ops[a];
                 uint64_t v = 1ull;
@@ -290,12 +291,12 @@ __global__ __launch_bounds__(kSegB) void seg_reduce_kernel(SegArgs sa, int is_si
 
 }  // namespace
 
-template <int KB>
+template <int KB, int MO>
 void launch_seg(const SegArgs& a, int is_signed, const AggSpec& spec, const OutSpec& os, hipStream_t s)
 {
     const size_t lds = (size_t)spec.nops * (kSegB + 1) * 8;
     lds::with_vlayout(spec, true, [&](auto vl) {
-        auto kern = seg_reduce_kernel<KB, decltype(vl)>;
+        auto kern = seg_reduce_kernel<KB, MO, decltype(vl)>;
         if (enable_dynamic_lds((const void*)kern) < lds) raise(EG_ERR_UNSUPPORTED, "segmented reduction slots too large");
         KernelTimer timer("segreduce", s);
         hipLaunchKernelGGL(kern, dim3(a.ntiles), dim3(kSegB), lds, s, a, is_signed, spec, os);

@@ -114,8 +114,9 @@ Result reduce_sorted(const Plan& plan, const void* sorted_keys, const AggSpec& s
     const int sg = plan.key.is_signed;
     const SegArgs sa{sorted_keys, perm, n, head_off.get<uint32_t>(), ntiles, bstate.get<unsigned long long>(),
                      bkey.get<unsigned long long>(), btrail.get<uint32_t>()};
-    if (kb == 4) launch_seg<4>(sa, sg, spec, os, s);
-    else launch_seg<8>(sa, sg, spec, os, s);
+    const bool few = spec.nops <= kSegFewOps;
+    if (kb == 4) (few ? launch_seg<4, kSegFewOps> : launch_seg<4, kMaxOps>)(sa, sg, spec, os, s);
+    else (few ? launch_seg<8, kSegFewOps> : launch_seg<8, kMaxOps>)(sa, sg, spec, os, s);
     hipLaunchKernelGGL(seg_tail_kernel, dim3((ntiles + 255) / 256), dim3(256), 0, s, ntiles,
                        (const uint32_t*)head_off.get<uint32_t>(), (const unsigned long long*)bstate.get<unsigned long long>(),
                        (const unsigned long long*)bkey.get<unsigned long long>(), (const uint32_t*)btrail.get<uint32_t>(),
