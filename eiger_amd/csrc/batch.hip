@@ -100,6 +100,7 @@ struct BPTile {
 constexpr int64_t kPTile = (int64_t)1 << 14;
 constexpr int kMaxPartBits = 12;
 constexpr int kPB = 256;  // threads of the partition-pass kernels
+constexpr int kPU = 4;    // rows a thread of theirs loads together
 
 struct BCItem {
     int32_t q;
@@ -151,6 +152,16 @@ __device__ __forceinline__ uint32_t part_of(uint64_t raw, uint32_t mask)
     return (uint32_t)dev::bit_mix<KB>(raw) & mask;
 }
 
+// One value of VB bytes (0: no value column; -1: any width, read at run time).
+template <int VB>
+__device__ __forceinline__ uint64_t load_value(const void* p, int vbytes, int64_t r)
+{
+    if constexpr (VB == 0) return 0ull;
+    else if constexpr (VB == 4) return ((const uint32_t*)p)[r];
+    else if constexpr (VB == 8) return ((const uint64_t*)p)[r];
+    else return dev::load_raw(p, vbytes, r);
+}
+
 template <int KB>
 __global__ __launch_bounds__(kPB) void bpart_hist_kernel(const BQuery* __restrict__ qs, const BPTile* __restrict__ tiles,
                                                          uint32_t* __restrict__ hist)
@@ -162,7 +173,14 @@ __global__ __launch_bounds__(kPB) void bpart_hist_kernel(const BQuery* __restric
     for (uint32_t i = threadIdx.x; i < P; i += kPB) h[i] = 0u;
     __syncthreads();
     const int64_t b = (int64_t)tt.t * kPTile, e = min(q.rows, b + kPTile);
-    for (int64_t r = b + threadIdx.x; r < e; r += kPB) atomicAdd(&h[part_of<KB>(dev::load_raw(q.keys, KB, r), mask)], 1u);
+    for (int64_t r0 = b + threadIdx.x; r0 < e; r0 += kPU * kPB) {
+        uint64_t raw[kPU];
+#pragma unroll
+        for (int u = 0; u < kPU; ++u) raw[u] = dev::load_raw(q.keys, KB, min(r0 + u * kPB, e - 1));
+#pragma unroll
+        for (int u = 0; u < kPU; ++u)
+            if (r0 + u * kPB < e) atomicAdd(&h[part_of<KB>(raw[u], mask)], 1u);
+    }
     __syncthreads();
     uint32_t* out = hist + q.hist_off + tt.t;
     for (uint32_t d = threadIdx.x; d < P; d += kPB) out[(int64_t)d * q.ntiles] = h[d];
@@ -220,8 +238,9 @@ __global__ __launch_bounds__(1024) void bpart_scan_kernel(const BQuery* __restri
 }
 
 // Moves every row of a tile to its partition in the scratch columns (the
-// order inside a partition is the order the LDS cursors hand out).
-template <int KB>
+// order inside a partition is the order the LDS cursors hand out).  VB: value
+// bytes as in load_value.
+template <int KB, int VB>
 __global__ __launch_bounds__(kPB) void bpart_scatter_kernel(const BQuery* __restrict__ qs, const BPTile* __restrict__ tiles,
                                                             const uint32_t* __restrict__ offs, void* __restrict__ skeys,
                                                             void* __restrict__ svals, int vbytes)
@@ -234,11 +253,25 @@ __global__ __launch_bounds__(kPB) void bpart_scatter_kernel(const BQuery* __rest
     for (uint32_t d = threadIdx.x; d < P; d += kPB) cur[d] = o[(int64_t)d * q.ntiles];
     __syncthreads();
     const int64_t b = (int64_t)tt.t * kPTile, e = min(q.rows, b + kPTile);
-    for (int64_t r = b + threadIdx.x; r < e; r += kPB) {
-        const uint64_t raw = dev::load_raw(q.keys, KB, r);
-        const int64_t dst = q.scratch_off + atomicAdd(&cur[part_of<KB>(raw, mask)], 1u);
-        dev::store_bytes(skeys, KB, dst, raw);
-        if (svals) dev::store_bytes(svals, vbytes, dst, dev::load_raw(q.vals, vbytes, r));
+    const void* keys = q.keys;
+    const void* vals = q.vals;
+    const int64_t base = q.scratch_off;
+    for (int64_t r0 = b + threadIdx.x; r0 < e; r0 += kPU * kPB) {
+        uint64_t raw[kPU], val[kPU];
+#pragma unroll
+        for (int u = 0; u < kPU; ++u) {
+            const int64_t r = min(r0 + u * kPB, e - 1);  // in bounds, masked below
+            raw[u] = dev::load_raw(keys, KB, r);
+            val[u] = load_value<VB>(vals, vbytes, r);
+        }
+#pragma unroll
+        for (int u = 0; u < kPU; ++u) {
+            if (r0 + u * kPB >= e) continue;
+            const int64_t dst = base + atomicAdd(&cur[part_of<KB>(raw[u], mask)], 1u);
+            dev::store_bytes(skeys, KB, dst, raw[u]);
+            if constexpr (VB == -1) dev::store_bytes(svals, vbytes, dst, val[u]);
+            else if constexpr (VB > 0) dev::store_bytes(svals, VB, dst, val[u]);
+        }
     }
 }
 
@@ -321,16 +354,6 @@ struct BConst {
     AggSpec spec;
     BOut bo;
 };
-
-// One value of VB bytes (0: no value column; -1: any width, read at run time).
-template <int VB>
-__device__ __forceinline__ uint64_t load_value(const void* p, int vbytes, int64_t r)
-{
-    if constexpr (VB == 0) return 0ull;
-    else if constexpr (VB == 4) return ((const uint32_t*)p)[r];
-    else if constexpr (VB == 8) return ((const uint64_t*)p)[r];
-    else return dev::load_raw(p, vbytes, r);
-}
 
 // Fewest of a step's first rows holding lane 0's key for a wave to keep that
 // key's partial states in registers (see hash_agg's rule).
@@ -641,10 +664,13 @@ void batch_default_tuning(eg_batch_tuning* t)
     t->radix_bits = 12;
 }
 
+// Value layout of the plan's kernels (see load_value).
+int value_layout(const BatchPlan& p) { return p.nv == 0 ? 0 : p.vbytes == 4 || p.vbytes == 8 ? p.vbytes : -1; }
+
 // The aggregation kernel for the plan's key and value widths.
 auto agg_kernel(const BatchPlan& p) -> decltype(&batch_agg_kernel<4, 0>)
 {
-    const int vb = p.nv == 0 ? 0 : p.vbytes == 4 || p.vbytes == 8 ? p.vbytes : -1;
+    const int vb = value_layout(p);
     if (p.kb == 4)
         return vb == 0 ? batch_agg_kernel<4, 0> : vb == 4 ? batch_agg_kernel<4, 4> : vb == 8 ? batch_agg_kernel<4, 8>
              : batch_agg_kernel<4, -1>;
@@ -856,7 +882,10 @@ void launch_partition_pass(BatchPlan& p, hipStream_t s)
     hipLaunchKernelGGL(bpart_scan_kernel, dim3((unsigned)p.n_pq), dim3(1024), 0, s, p.qs.get<BQuery>(),
                        p.pqs.get<int32_t>(), p.hist.get<uint32_t>());
     EG_LAUNCH_CHECK();
-    hipLaunchKernelGGL(bpart_scatter_kernel<KB>, dim3((unsigned)p.n_ptiles), dim3(kPB), 0, s, p.qs.get<BQuery>(),
+    const int vb = value_layout(p);
+    auto scatter = vb == 0 ? bpart_scatter_kernel<KB, 0> : vb == 4 ? bpart_scatter_kernel<KB, 4>
+                 : vb == 8 ? bpart_scatter_kernel<KB, 8> : bpart_scatter_kernel<KB, -1>;
+    hipLaunchKernelGGL(scatter, dim3((unsigned)p.n_ptiles), dim3(kPB), 0, s, p.qs.get<BQuery>(),
                        p.ptiles.get<BPTile>(), (const uint32_t*)p.hist.get<uint32_t>(), p.skeys.get(), p.svals.get(),
                        p.vbytes);
     EG_LAUNCH_CHECK();
