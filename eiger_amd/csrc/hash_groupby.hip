@@ -97,8 +97,12 @@ void aggregate(bool vec, const HashTuning& t, const KeyDesc& key, int64_t n, con
     HashLaunch h = prepare_hash_agg<KB>(vec, t, n, spec, L, use_jit);
     unsigned long long* priv = nullptr;
     if (scratch && L.cr > 0 && h.grid >= kPrivMinBlocks) {
-        *scratch = DevBuf((size_t)h.grid * (size_t)(1 + spec.nops) * (L.cr + 1) * 8, s);
-        priv = scratch->get<unsigned long long>();
+        try {
+            *scratch = DevBuf((size_t)h.grid * (size_t)(1 + spec.nops) * (L.cr + 1) * 8, s);
+            priv = scratch->get<unsigned long long>();
+        } catch (const std::bad_alloc&) {
+            // no room (a small memory pool): flush with atomics
+        }
     }
     launch_hash_agg<KB>(h, key, n, spec, gt, L, priv, s);
     if (!priv) return;
