@@ -145,3 +145,37 @@ def test_hash_tables_of_many_workgroups_merged(dtype, d, n):
         for bound in (len(exp[0]), max(1, len(exp[0]) // 3)):
             got = sorted_by_key(run(G.hash_groupby, keys, [vals, f], reqs, G.groupby_hint(groups_upper_bound=bound)))
             assert_same(got, exp)
+
+
+@pytest.mark.parametrize("n", [1, 1023, 1025, 4096, 4097])
+@pytest.mark.parametrize("ktype", [np.int32, np.int64, np.uint8, np.float32])
+def test_tiny_inputs_in_one_workgroup(n, ktype):
+    """Row counts around one workgroup's rows, one group to a group a row, 1-
+    to 8-byte values, few and many states (more than its LDS holds), the keys
+    whose encodings are the empty word, a key every row holds."""
+    rng = np.random.default_rng(n)
+    for d in (1, 7, n):
+        keys = rng.integers(0, max(1, min(d, 250)) if ktype == np.uint8 else d, n).astype(ktype)
+        if np.dtype(ktype).kind == "i" and n > 3 and d > 1:
+            keys[1], keys[2] = np.iinfo(ktype).min, np.iinfo(ktype).max
+        vals = [rng.integers(-100, 100, n).astype(t) for t in (np.int64, np.int8, np.int16, np.float64)]
+        for reqs in ([(0, A.SUM), (-1, A.COUNT_ALL)], [(1, A.MIN), (2, A.MAX)],
+                     [(i, k) for i in range(4) for k in (A.SUM, A.MIN, A.MAX)]):
+            exp = sorted_by_key(O.groupby(keys, vals, reqs))
+            got = sorted_by_key(run(G.hash_groupby, keys, vals, reqs, G.groupby_hint(groups_upper_bound=max(1, d // 2))))
+            assert_same(got, exp, 1e-9)
+
+
+@pytest.mark.parametrize("bound", [300, 100_000, 390_000, 1_100_000])
+def test_partition_counts_around_the_one_launch_unit_list(bound):
+    """Bounds that give a few, about 100, 256 (one digit pass, fuller tables)
+    and more than 512 partitions, over keys far fewer than the bound with one
+    key that most rows hold (its partition is sliced)."""
+    n = 1_200_007
+    keys = O.gen_keys_uniform(n, 20_011, seed=bound)
+    keys[np.random.default_rng(3).random(n) < 0.6] = 77
+    vals = O.gen_values(n, O.VAL_UNIFORM_I64, np.int64, seed=4, stream_id=2)
+    reqs = [(0, A.SUM), (0, A.MIN), (-1, A.COUNT_ALL)]
+    exp = sorted_by_key(O.groupby(keys, [vals], reqs))
+    for fn in (G.partition_groupby, G.partition_groupby_gfur):
+        assert_same(sorted_by_key(run(fn, keys, [vals], reqs, G.groupby_hint(groups_upper_bound=min(bound, n - 1)))), exp)
