@@ -25,7 +25,8 @@ void timing_query(const char* name, int64_t* launches, double* total_ms);
 void zipf_cdf(double* cdf, int64_t distinct, double s);
 Result run_sort(const Plan& plan, const eg_groupby_hint& hint, bool gfur, hipStream_t s);
 Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream_t s);
-int partition_passes(const Plan& plan, int64_t group_bound);  // its radix passes at this bound
+// Its radix passes at this bound, and the rows an average partition has.
+int partition_passes(const Plan& plan, int64_t group_bound, int64_t* rows_per_part);
 bool mlp_select(const void* keys, int32_t key_type, int64_t rows, int64_t group_bound, int nops, int value_bytes,
                 hipStream_t s, int32_t* algo, int64_t* card_est, float* singletons);
 int64_t ndv_approx(const void* data, int32_t type, int64_t n, hipStream_t s);
@@ -436,8 +437,12 @@ int groupby_entry(Entry entry, const eg_column_view* keys, int64_t num_keys,
                     // 16.7M groups were cut into 32768 partitions for the row
                     // count as bound: 2.98 -> 2.75 ms).  With one, and the
                     // partition strategy, only where a tighter bound could
-                    // save a radix pass or two digit bits of two passes: else
-                    // it costs more (0.25 ms per 2^28 rows) than it saves.
+                    // save a radix pass, two digit bits of two passes, or
+                    // where the partitions are so small (16384 rows) that
+                    // fewer of them make a faster unit kernel (2^28 rows, Zipf
+                    // 1.0, 2^26 as bound for 30M groups: 8.0 ms without the
+                    // estimate, 7.4 with it): else it costs more (0.25 ms per
+                    // 2^28 rows) than it saves.
                     // Below 2^24 rows the pass and its synchronisation would
                     // cost more than the tighter sizing saves; the model's
                     // estimate stays within 1.34x of the true count on every
@@ -446,9 +451,11 @@ int groupby_entry(Entry entry, const eg_column_view* keys, int64_t num_keys,
                     const bool known = h.groups_upper_bound > 0 && h.groups_upper_bound < plan.rows;
                     const int64_t caller = known ? h.groups_upper_bound : plan.rows;
                     learned_bound = std::min<int64_t>(caller, card + card + card / 2 + 1024);
-                    const int passes = known && a == EG_ALGO_PARTITION ? partition_passes(plan, caller) : 0;
-                    if (plan.rows >= ((int64_t)1 << 24) && passes > 0 && passes == partition_passes(plan, learned_bound) &&
-                        (passes == 1 || 4 * learned_bound >= caller)) {
+                    int64_t part_rows = 0;
+                    const int passes = known && a == EG_ALGO_PARTITION ? partition_passes(plan, caller, &part_rows) : 0;
+                    if (plan.rows >= ((int64_t)1 << 24) && passes > 0 &&
+                        passes == partition_passes(plan, learned_bound, nullptr) &&
+                        (passes == 1 || (4 * learned_bound >= caller && part_rows >= 16384))) {
                         learned_bound = caller;
                     } else if ((learned_bound < caller || !known) && singletons > 0.25f &&
                                plan.rows >= ((int64_t)1 << 24)) {

@@ -293,10 +293,12 @@ PartGeometry part_geometry(int nops, int kb, int64_t bound)
 
 }  // namespace
 
-int partition_passes(const Plan& plan, int64_t group_bound)
+int partition_passes(const Plan& plan, int64_t group_bound, int64_t* rows_per_part)
 {
     const int64_t bound = std::max<int64_t>(1, std::min<int64_t>(group_bound, plan.rows));
-    return (part_geometry(plan.spec.nops, plan.key.bytes, bound).bits + max_digit_bits() - 1) / max_digit_bits();
+    const int bits = part_geometry(plan.spec.nops, plan.key.bytes, bound).bits;
+    if (rows_per_part) *rows_per_part = plan.rows >> bits;
+    return (bits + max_digit_bits() - 1) / max_digit_bits();
 }
 
 Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream_t s)
