@@ -359,7 +359,10 @@ __device__ __forceinline__ void hash_agg(const KeyDesc& key, int64_t n, const Ag
         const bool sp = lds_row<OPS, KB, NV>(tab, use_lds, r_mask, lane, key, spec, kraw, cv, valid, probe_limit, peel_min, hot);
         if (__ballot(sp) != 0ull) hbm_rows<OPS, KB, NV>(gt, key, spec, sp, kraw, cv, hbm_peel, ins, hot);
     }
-    if (use_lds) flush_lds<OPS>(tab, gt, key, spec, rep_log2, r_mask, ins, priv);
+    // opaque here, so nothing of the flush is computed ahead and kept in scalar
+    // registers (spilled ones slow the row loop) while rows are read
+    asm volatile("" : "+s"(rep_log2));
+    if (use_lds) flush_lds<OPS>(tab, gt, key, spec, rep_log2, (1 << rep_log2) - 1, ins, priv);
     gt_count_inserts(gt, ins);
 }
 
