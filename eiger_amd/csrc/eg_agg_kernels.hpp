@@ -360,7 +360,8 @@ __device__ __forceinline__ void hash_agg(const KeyDesc& key, int64_t n, const Ag
         if (__ballot(sp) != 0ull) hbm_rows<OPS, KB, NV>(gt, key, spec, sp, kraw, cv, hbm_peel, ins, hot);
     }
     // opaque here, so nothing of the flush is computed ahead and kept in scalar
-    // registers (spilled ones slow the row loop) while rows are read
+    // registers while rows are read (53 of them spilled instead of 63; no
+    // difference in time: 0.88-0.89 ms for 2^28 rows of 16 groups)
     asm volatile("" : "+s"(rep_log2));
     if (use_lds) flush_lds<OPS>(tab, gt, key, spec, rep_log2, (1 << rep_log2) - 1, ins, priv);
     gt_count_inserts(gt, ins);

@@ -81,9 +81,9 @@ void launch_compact(const GTable& gt, const OutSpec& os, unsigned long long* cou
 
 // Grids of fewer blocks flush straight into the HBM table.
 constexpr int64_t kPrivMinBlocks = 16;
-// So do bounds of fewer groups: their few atomics cost less than a launch
-// that waits for every table (2^28 rows, 16 groups: 0.79-0.81 ms a call
-// flushed, 0.85-0.90 stored and merged).
+// So do bounds of fewer groups, which spares them the merge's launch and its
+// buffer; the time is the same either way (2^28 rows, 16 groups: 0.88-0.89 ms
+// a call flushed, 0.85-0.90 stored and merged).
 constexpr int64_t kPrivMinGroups = 64;
 
 // The aggregation of n rows into gt.  `scratch` (optional): where the blocks'
