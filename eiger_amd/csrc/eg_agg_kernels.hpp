@@ -61,20 +61,20 @@ __device__ __forceinline__ void merge_replicas(LdsTable<KB>& tab, const GTable& 
 }
 
 // Ends a block's aggregation: its groups go to the HBM table with atomics,
-// or (priv) its table is stored as it stands for table_merge to combine.
+// or (STORE) its table is stored as it stands at priv for table_merge to combine.
 // Every block of a large grid holds the same groups, so the atomics of all
 // blocks meet on the same few lines: 256 blocks of 1024 groups and two states
 // took 250 us, the stored tables and their merge 25.
 // Words of a stored table: cr + 1 keys (64-bit encoding, 0 = empty; the side
 // slot last: its encoding, or 1 where that is 0), then cr + 1 states per op.
-template <class OPS, int KB>
+template <class OPS, bool STORE, int KB>
 __device__ __forceinline__ void flush_lds(LdsTable<KB>& tab, const GTable& gt, const KeyDesc& key, const AggSpec& spec,
                           int rep_log2, int r_mask, uint32_t& ins, unsigned long long* priv)
 {
     using KT = typename LdsKey<KB>::T;
     __syncthreads();
     merge_replicas<OPS>(tab, gt, key, spec, rep_log2, r_mask, ins);
-    if (priv) {
+    if constexpr (STORE) {
         const int nops = OPS::n(spec);
         unsigned long long* out = priv + (size_t)blockIdx.x * (size_t)(1 + nops) * (tab.cr + 1);
         for (int s = threadIdx.x; s <= tab.cr; s += blockDim.x) {
@@ -190,7 +190,12 @@ __device__ constexpr int priv_ops()
 // hash kernel to keep that key in registers.
 constexpr int kPrivLanes = 8;
 
-template <int KB, class VL, class OPS>
+// STORE: the block's table ends at `priv` (see flush_lds).  A kernel of its own:
+// with both endings in one kernel and the choice at run time, the calls that
+// flush lost 4-8% to the code around the row loop, whose source is the same
+// (2^28 rows, five states: 16 groups 0.79 -> 0.85 ms, 2^22 keys at Zipf 1.5
+// 2.42 -> 2.54 ms).
+template <int KB, class VL, class OPS, bool STORE>
 __device__ __forceinline__ void hash_agg(const KeyDesc& key, int64_t n, const AggSpec& spec, const GTable& gt,
                                          int cr, int rep_log2, int probe_limit, int peel_min,
                                          unsigned long long* priv)
@@ -359,11 +364,7 @@ __device__ __forceinline__ void hash_agg(const KeyDesc& key, int64_t n, const Ag
         const bool sp = lds_row<OPS, KB, NV>(tab, use_lds, r_mask, lane, key, spec, kraw, cv, valid, probe_limit, peel_min, hot);
         if (__ballot(sp) != 0ull) hbm_rows<OPS, KB, NV>(gt, key, spec, sp, kraw, cv, hbm_peel, ins, hot);
     }
-    // opaque here, so nothing of the flush is computed ahead and kept in scalar
-    // registers while rows are read (53 of them spilled instead of 63; no
-    // difference in time: 0.88-0.89 ms for 2^28 rows of 16 groups)
-    asm volatile("" : "+s"(rep_log2));
-    if (use_lds) flush_lds<OPS>(tab, gt, key, spec, rep_log2, (1 << rep_log2) - 1, ins, priv);
+    if (use_lds) flush_lds<OPS, STORE>(tab, gt, key, spec, rep_log2, r_mask, ins, priv);
     gt_count_inserts(gt, ins);
 }
 

@@ -1,5 +1,5 @@
 // eg_hash_launch.hpp -- launch of the hash aggregation kernel: one translation
-// unit instantiates it per key width (hash_agg*.hip).
+// unit instantiates it per key width and ending (hash_agg*.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -21,12 +21,13 @@ struct HashLaunch {
 
 // Picks the compiled value layout (vector loads for up to two 4/8-byte
 // columns on 16-byte aligned data, else typed loads), the specialised kernel
-// when use_jit and it is loaded, and the grid.
-template <int KB>
+// when use_jit and it is loaded, and the grid.  STORE: the kernel whose blocks
+// store their tables instead of flushing them (see agg::flush_lds).
+template <int KB, bool STORE>
 HashLaunch prepare_hash_agg(bool vec, const HashTuning& t, int64_t n, const AggSpec& spec, const HashLayout& L,
                             bool use_jit);
 
-// priv: one stored table per block of h.grid (see agg::flush_lds), or nullptr.
+// priv: room for one stored table per block of h.grid (STORE kernels).
 template <int KB>
 void launch_hash_agg(const HashLaunch& h, const KeyDesc& key, int64_t n, const AggSpec& spec, const GTable& gt,
                      const HashLayout& L, unsigned long long* priv, hipStream_t s);

@@ -12,18 +12,18 @@ namespace eg {
 namespace {
 using agg::max_block;
 
-template <int KB, class VL>
+template <int KB, class VL, bool STORE>
 __global__ __launch_bounds__(max_block<VL::NV>()) void hash_agg_kernel(KeyDesc key, int64_t n, AggSpec spec,
                                                                         GTable gt, int cr, int rep_log2,
                                                                         int probe_limit, int peel_min,
                                                                         unsigned long long* priv)
 {
-    agg::hash_agg<KB, VL, dev::RtOps>(key, n, spec, gt, cr, rep_log2, probe_limit, peel_min, priv);
+    agg::hash_agg<KB, VL, dev::RtOps, STORE>(key, n, spec, gt, cr, rep_log2, probe_limit, peel_min, priv);
 }
 
 }  // namespace
 
-template <int KB>
+template <int KB, bool STORE>
 HashLaunch prepare_hash_agg(bool vec, const HashTuning& t, int64_t n, const AggSpec& spec, const HashLayout& L,
                             bool use_jit)
 {
@@ -31,11 +31,12 @@ HashLaunch prepare_hash_agg(bool vec, const HashTuning& t, int64_t n, const AggS
     HashLaunch h;
     lds::with_vlayout(spec, vec, [&](auto vl) {
         using VL = decltype(vl);
-        h.kern = hash_agg_kernel<KB, VL>;
+        h.kern = hash_agg_kernel<KB, VL, STORE>;
         enable_dynamic_lds((const void*)h.kern);
         h.block = std::min(t.block, max_block<VL::NV>());
         // the kernel with this request's ops compiled in, once it is available
-        if (use_jit) h.fn = jit::lookup(jit::Kind::HASH_AGG, KB, jit::vlayout_name<VL>(), spec, n);
+        const jit::Kind kind = STORE ? jit::Kind::HASH_AGG_STORE : jit::Kind::HASH_AGG;
+        if (use_jit) h.fn = jit::lookup(kind, KB, jit::vlayout_name<VL>(), spec, n);
     });
     const int64_t tile = (int64_t)h.block * lds::kRows;
     const int64_t want = (n + tile - 1) / tile;

@@ -10,7 +10,8 @@
 namespace eg {
 namespace jit {
 
-enum class Kind { HASH_AGG, PART_AGG, PART_AGG_GATHER };
+// HASH_AGG and HASH_AGG_STORE are two kernels of one module, compiled together.
+enum class Kind { HASH_AGG, HASH_AGG_STORE, PART_AGG, PART_AGG_GATHER };
 
 // The kernel specialised for (kind, key bytes, value layout type name, ops of
 // `spec`), or nullptr while it is not available: JIT off, `rows` below the

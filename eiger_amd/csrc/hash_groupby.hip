@@ -16,8 +16,15 @@
 //      cannot find a slot within `probe_limit` probes spills to the HBM
 //      table.  Hot keys (many lanes of a wave on one group) are combined by
 //      the wave first (eg_atomics.hpp) so one atomic per state is issued.
-//   2. hash_compact_kernel: scans the HBM table and writes the final key and
+//      The finished table goes into the HBM table with atomics, or, where
+//      that would cost more (store_pays), is stored as it stands.
+//   2. hash_merge_kernel, after stored tables: combines the same slots of
+//      every workgroup's table and adds the result to the HBM table.
+//   3. hash_compact_kernel: scans the HBM table and writes the final key and
 //      output columns at wave-aggregated positions.
+//
+// Up to 4096 rows one workgroup does all of it in one launch, straight to the
+// outputs (hash_tiny_kernel).
 //
 // The HBM table stores slots of W = 2^k 64-bit words [enc key | states...]
 // (AoS, so a random update touches one cache line).  The all-zero word is
@@ -79,44 +86,52 @@ void launch_compact(const GTable& gt, const OutSpec& os, unsigned long long* cou
     EG_LAUNCH_CHECK();
 }
 
-// Grids of fewer blocks flush straight into the HBM table.
-constexpr int64_t kPrivMinBlocks = 16;
-// So do bounds of fewer groups, which spares them the merge's launch and its
-// buffer; the time is the same either way (2^28 rows, 16 groups: 0.88-0.89 ms
-// a call flushed, 0.85-0.90 stored and merged).
-constexpr int64_t kPrivMinGroups = 64;
+// Whether the workgroups' tables are better stored and merged than flushed
+// with atomics.  A flush costs one atomic per state for each group a block
+// holds, serialised across the blocks on the groups' lines; storing costs the
+// merge's launch (5 us) and 2-8% of the row loop, whose kernel is the slower
+// one.  Measured on both sides, two and five states, us flushed / stored:
+// 2^16 rows, 200 groups 45/48, 400 54/50; 2^18, 64 47/48, 128 51/49;
+// 2^20, 16 52/49, 1000 306/60; 2^26, 64 248/244, 128 274/246; 2^28 (five
+// states), 16 766/832, 200 789/796, 400 891/808.
+bool store_pays(int64_t rows, int64_t bound)
+{
+    const int64_t tiles = (rows + 4095) / 4096;
+    const int64_t blocks = std::min<int64_t>(tiles, device_info().num_cus);
+    return blocks * bound >= 6400 + tiles;
+}
 
 // The aggregation of n rows into gt.  `scratch` (optional): where the blocks'
-// tables may be stored, allocated here; without it (callers that must not
-// allocate), and where the group bound is above twice the LDS slots (the
-// tables then hold different keys: 3M rows in 400k groups 329 us flushed, 622 us
-// stored and merged), every block flushes into gt with atomics.  use_jit: take the
-// specialised kernel once it is loaded (loading a module allocates device
-// memory for its code, so callers that must not allocate pass false and
-// always run the generic kernel).
+// tables are stored, allocated here; without it (callers that must not
+// allocate), or without room for it, every block flushes into gt with atomics.
+// use_jit: take the specialised kernel once it is loaded (loading a module
+// allocates device memory for its code, so callers that must not allocate pass
+// false and always run the generic kernel).
 template <int KB>
 void aggregate(bool vec, const HashTuning& t, const KeyDesc& key, int64_t n, const AggSpec& spec, const GTable& gt,
                const HashLayout& L, hipStream_t s, bool use_jit, DevBuf* scratch)
 {
-    HashLaunch h = prepare_hash_agg<KB>(vec, t, n, spec, L, use_jit);
-    unsigned long long* priv = nullptr;
-    if (scratch && L.cr > 0 && h.grid >= kPrivMinBlocks) {
+    if (scratch && L.cr > 0) {
+        const HashLaunch h = prepare_hash_agg<KB, true>(vec, t, n, spec, L, use_jit);
         try {
             *scratch = DevBuf((size_t)h.grid * (size_t)(1 + spec.nops) * (L.cr + 1) * 8, s);
-            priv = scratch->get<unsigned long long>();
         } catch (const std::bad_alloc&) {
             // no room (a small memory pool): flush with atomics
         }
+        if (unsigned long long* priv = scratch->get<unsigned long long>()) {
+            launch_hash_agg<KB>(h, key, n, spec, gt, L, priv, s);
+            const int grid = (L.cr + 1 + agg::kMergeSlots - 1) / agg::kMergeSlots;
+            const size_t lds = (size_t)lds_table_words(spec.nops, agg::kMergeCr, 0, 8) * 8;
+            if (enable_dynamic_lds((const void*)hash_merge_kernel) < lds) raise(EG_ERR_DEVICE, "hash merge: LDS");
+            KernelTimer timer("hash_merge", s);
+            hipLaunchKernelGGL(hash_merge_kernel, dim3((unsigned)grid), dim3(agg::kMergeBlock), lds, s,
+                               (const unsigned long long*)priv, (int)h.grid, L.cr, spec, gt, KB == 8 ? 1 : 0);
+            EG_LAUNCH_CHECK();
+            return;
+        }
     }
-    launch_hash_agg<KB>(h, key, n, spec, gt, L, priv, s);
-    if (!priv) return;
-    const int grid = (L.cr + 1 + agg::kMergeSlots - 1) / agg::kMergeSlots;
-    const size_t lds = (size_t)lds_table_words(spec.nops, agg::kMergeCr, 0, 8) * 8;
-    if (enable_dynamic_lds((const void*)hash_merge_kernel) < lds) raise(EG_ERR_DEVICE, "hash merge: LDS");
-    KernelTimer timer("hash_merge", s);
-    hipLaunchKernelGGL(hash_merge_kernel, dim3((unsigned)grid), dim3(agg::kMergeBlock), lds, s,
-                       (const unsigned long long*)priv, (int)h.grid, L.cr, spec, gt, KB == 8 ? 1 : 0);
-    EG_LAUNCH_CHECK();
+    const HashLaunch h = prepare_hash_agg<KB, false>(vec, t, n, spec, L, use_jit);
+    launch_hash_agg<KB>(h, key, n, spec, gt, L, nullptr, s);
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
@@ -306,7 +321,9 @@ Result run_hash(const Plan& plan, int64_t group_bound, hipStream_t s, const Hash
     for (;;) {
         HbmTable ht(slots, W, s);
         DevBuf scratch;
-        DevBuf* stored = bound > kPrivMinGroups && bound <= 2 * (int64_t)L.cr ? &scratch : nullptr;
+        // bounds above twice the LDS slots flush: the tables then hold different
+        // keys (3M rows in 400k groups 329 us flushed, 622 stored and merged)
+        DevBuf* stored = bound <= 2 * (int64_t)L.cr && store_pays(n, bound) ? &scratch : nullptr;
         if (KB == 4) aggregate<4>(vec, t, plan.key, n, plan.spec, ht.gt, L, s, true, stored);
         else aggregate<8>(vec, t, plan.key, n, plan.spec, ht.gt, L, s, true, stored);
         Result eres;

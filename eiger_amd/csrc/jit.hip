@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hiprtc.h>
 
+#include <array>
 #include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
@@ -52,7 +53,7 @@ struct Entry {
     std::string arch;
     std::vector<char> code;
     std::string log;
-    std::map<int, hipFunction_t> fn;  // per device
+    std::map<int, std::array<hipFunction_t, 2>> fn;  // per device; [1]: a hash module's storing kernel
 };
 
 struct Runtime {
@@ -256,21 +257,31 @@ std::string out_list(const OutSpec& os)
     return o.str();
 }
 
+bool is_hash(Kind kind) { return kind == Kind::HASH_AGG || kind == Kind::HASH_AGG_STORE; }
+
+// The kernel's name in its module.
+const char* kernel_name(Kind kind)
+{
+    return kind == Kind::HASH_AGG ? "eg_jit_hash_agg" : kind == Kind::HASH_AGG_STORE ? "eg_jit_hash_agg_store"
+                                                                                     : "eg_jit_part_agg";
+}
+
 std::string make_source(Kind kind, int kb, const std::string& vl, const AggSpec& spec, const OutSpec* os)
 {
     std::ostringstream o;
     o << "#include \"eg_agg_kernels.hpp\"\n"
       << "using JitOps = eg::dev::FixOps<" << op_list(spec) << ">;\n"
       << "using JitVL = " << vl << ";\n";
-    if (kind != Kind::HASH_AGG)
+    if (!is_hash(kind))
         o << "using JitOuts = " << (os ? "eg::dev::FixOuts<" + out_list(*os) + ">" : std::string("eg::dev::RtOuts"))
           << ";\n";
-    if (kind == Kind::HASH_AGG) {
-        o << "extern \"C\" __global__ __launch_bounds__(eg::agg::max_block<JitVL::NV>()) void eg_jit_hash_agg("
-             "eg::KeyDesc key, int64_t n, eg::AggSpec spec, eg::GTable gt, int cr, int rep_log2, "
-             "int probe_limit, int peel_min, unsigned long long* priv)\n{\n"
-          << "    eg::agg::hash_agg<" << kb
-          << ", JitVL, JitOps>(key, n, spec, gt, cr, rep_log2, probe_limit, peel_min, priv);\n}\n";
+    if (is_hash(kind)) {
+        for (const Kind k : {Kind::HASH_AGG, Kind::HASH_AGG_STORE})
+            o << "extern \"C\" __global__ __launch_bounds__(eg::agg::max_block<JitVL::NV>()) void " << kernel_name(k)
+              << "(eg::KeyDesc key, int64_t n, eg::AggSpec spec, eg::GTable gt, int cr, int rep_log2, "
+                 "int probe_limit, int peel_min, unsigned long long* priv)\n{\n"
+              << "    eg::agg::hash_agg<" << kb << ", JitVL, JitOps, " << (k == Kind::HASH_AGG_STORE ? "true" : "false")
+              << ">(key, n, spec, gt, cr, rep_log2, probe_limit, peel_min, priv);\n}\n";
     } else {
         o << "extern \"C\" __global__ __launch_bounds__(eg::agg::kPBMax, 8) void eg_jit_part_agg(eg::KeyDesc key, "
              "eg::AggSpec spec, const int64_t* perm, const eg::agg::Unit* units, eg::GTable gt, eg::OutSpec os, "
@@ -331,12 +342,18 @@ hipFunction_t lookup(Kind kind, int kb, const std::string& vl, const AggSpec& sp
     }
     Entry* e = it->second.get();
     if (e->state != Entry::READY) return nullptr;
+    const int which = kind == Kind::HASH_AGG_STORE ? 1 : 0;
     auto f = e->fn.find(dev);
-    if (f != e->fn.end()) return f->second;
+    if (f != e->fn.end()) return f->second[which];
     hipModule_t mod = nullptr;
-    hipFunction_t fn = nullptr;
-    if (hipModuleLoadData(&mod, e->code.data()) != hipSuccess ||
-        hipModuleGetFunction(&fn, mod, kind == Kind::HASH_AGG ? "eg_jit_hash_agg" : "eg_jit_part_agg") != hipSuccess) {
+    std::array<hipFunction_t, 2> fn{};
+    bool ok = hipModuleLoadData(&mod, e->code.data()) == hipSuccess;
+    if (is_hash(kind))
+        ok = ok && hipModuleGetFunction(&fn[0], mod, kernel_name(Kind::HASH_AGG)) == hipSuccess &&
+             hipModuleGetFunction(&fn[1], mod, kernel_name(Kind::HASH_AGG_STORE)) == hipSuccess;
+    else
+        ok = ok && hipModuleGetFunction(&fn[0], mod, kernel_name(kind)) == hipSuccess;
+    if (!ok) {
         (void)hipGetLastError();
         e->state = Entry::FAILED;
         ++r.failed;
@@ -345,7 +362,7 @@ hipFunction_t lookup(Kind kind, int kb, const std::string& vl, const AggSpec& sp
     }
     e->fn.emplace(dev, fn);  // modules stay loaded until the process ends
     arm_exit_join();
-    return fn;
+    return fn[which];
 }
 
 bool compile_check(Kind kind, int kb, const std::string& vl, const AggSpec& spec, const std::string& arch,
@@ -385,7 +402,7 @@ bool launch(hipFunction_t f, unsigned grid, unsigned block, size_t lds, hipStrea
         // never offered again: mark every entry holding this function failed
         for (auto& kv : r.cache)
             for (auto& df : kv.second->fn)
-                if (df.second == f) {
+                if (df.second[0] == f || df.second[1] == f) {
                     kv.second->state = Entry::FAILED;
                     ++r.failed;
                 }

@@ -129,9 +129,9 @@ def test_fused_keys_around_32_bits(bits, algo):
 @pytest.mark.parametrize("d", [1, 16, 1000, 7999, 16_400])
 @pytest.mark.parametrize("n", [16 * 4096, 200_003])
 def test_hash_tables_of_many_workgroups_merged(dtype, d, n):
-    """Grids of 16 workgroups and more store their LDS tables and merge them:
-    one group to twice the LDS slots, with the keys whose encodings are the
-    empty word, and undersized bounds."""
+    """Grids of 16 and 49 workgroups, whose LDS tables are flushed with atomics
+    (few groups, and 16,400, above twice the LDS slots) or stored and merged:
+    the keys whose encodings are the empty word, and undersized bounds."""
     rng = np.random.default_rng(d)
     info = np.iinfo(dtype)
     keys = rng.integers(0, d, n).astype(dtype)
@@ -145,6 +145,37 @@ def test_hash_tables_of_many_workgroups_merged(dtype, d, n):
         for bound in (len(exp[0]), max(1, len(exp[0]) // 3)):
             got = sorted_by_key(run(G.hash_groupby, keys, [vals, f], reqs, G.groupby_hint(groups_upper_bound=bound)))
             assert_same(got, exp)
+
+
+@pytest.mark.parametrize("n,bound,d,stored", [
+    (65_536, 400, 400, False), (65_536, 401, 401, True),        # 16 tiles: 16 * bound against 6400 + 16
+    (1 << 20, 25, 25, False), (1 << 20, 26, 20, True),          # 256 tiles: one a compute unit
+    ((1 << 20) + 1, 26, 3, False), ((1 << 20) + 1, 27, 1, True),
+    (200_003, 16_272, 16_000, True), (200_003, 16_273, 16_000, False),  # twice the LDS slots of two states
+])
+def test_hash_tables_stored_or_flushed(n, bound, d, stored):
+    """Both sides of the lines between flushing and storing the workgroups'
+    tables, by the kernels that ran; generic and specialised kernels."""
+    rng = np.random.default_rng(bound)
+    keys = rng.integers(0, d, n).astype(np.int32)
+    vals = rng.integers(-1000, 1000, n).astype(np.int64)
+    reqs = [(0, A.SUM), (-1, A.COUNT_ALL)]
+    exp = sorted_by_key(O.groupby(keys, [vals], reqs))
+    before = G.jit_stats()
+    try:
+        for mode in (G.jit_mode.OFF, G.jit_mode.SYNC):
+            G.jit_configure(mode, 0)
+            G.kernel_timing(True)
+            G.kernel_timing_reset()
+            l0 = G.jit_stats()["launches"]
+            got = sorted_by_key(run(G.hash_groupby, keys, [vals], reqs, G.groupby_hint(groups_upper_bound=bound)))
+            assert_same(got, exp)
+            assert G.kernel_time("hash_merge")[0] == (1 if stored else 0)
+            assert G.jit_stats()["launches"] - l0 == (0 if mode == G.jit_mode.OFF else 1)
+    finally:
+        G.kernel_timing(False)
+        G.kernel_timing_reset()
+        G.jit_configure(before["mode"], before["min_rows"])
 
 
 @pytest.mark.parametrize("n", [1, 1023, 1025, 4096, 4097])
