@@ -320,20 +320,20 @@ Result run_hash(const Plan& plan, int64_t group_bound, hipStream_t s, const Hash
     const bool early = bound <= kEarlyOutputRows;
     for (;;) {
         HbmTable ht(slots, W, s);
+        // before the stored tables, which take only room that is left
+        Result eres;
+        OutSpec eos;
+        if (early) alloc_outputs(plan, bound, s, eres, eos);
         DevBuf scratch;
         // bounds above twice the LDS slots flush: the tables then hold different
         // keys (3M rows in 400k groups 329 us flushed, 622 stored and merged)
         DevBuf* stored = bound <= 2 * (int64_t)L.cr && store_pays(n, bound) ? &scratch : nullptr;
         if (KB == 4) aggregate<4>(vec, t, plan.key, n, plan.spec, ht.gt, L, s, true, stored);
         else aggregate<8>(vec, t, plan.key, n, plan.spec, ht.gt, L, s, true, stored);
-        Result eres;
-        OutSpec eos;
-        if (early) {
-            alloc_outputs(plan, bound, s, eres, eos);
-            launch_compact(ht.gt, eos, ht.gt.meta + 3, s, bound);  // meta[3]: zeroed with the table
-        }
+        if (early) launch_compact(ht.gt, eos, ht.gt.meta + 3, s, bound);  // meta[3]: zeroed with the table
         int64_t meta[3];
         ht.read_meta(meta, s);
+        scratch = DevBuf();  // for the outputs allocated below, or the retry's table
         if (meta[2] != 0) {
             // The table filled up: the group bound was too small.  Retry with a
             // table sized for every row being its own group.
