@@ -121,18 +121,19 @@ __global__ __launch_bounds__(256) void part_compact_kernel(GTable gt, OutSpec os
 }
 
 // Units from the partition boundaries, on the device: a partition of at most
-// `slice` rows is one unit, a larger one ceil(rows / slice) sliced units.
+// `whole` rows is one unit, a larger one ceil(rows / slice) sliced units
+// (slice <= whole).
 // units_count_kernel counts each partition's units (cnt) and the sliced
 // partitions (meta[0]); after an exclusive scan of cnt (pre),
 // units_fill_kernel writes them and the unit total (meta[1]).
-__global__ __launch_bounds__(256) void units_count_kernel(const int64_t* __restrict__ offs, int64_t P, int64_t slice,
-                                                          uint32_t* __restrict__ cnt, unsigned long long* meta)
+__global__ __launch_bounds__(256) void units_count_kernel(const int64_t* __restrict__ offs, int64_t P, int64_t whole,
+                                                          int64_t slice, uint32_t* __restrict__ cnt, unsigned long long* meta)
 {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= P) return;
     const int64_t rows = offs[p + 1] - offs[p];
-    cnt[p] = rows <= 0 ? 0u : rows <= slice ? 1u : (uint32_t)((rows + slice - 1) / slice);
-    if (rows > slice) atomicAdd(&meta[0], 1ull);
+    cnt[p] = rows <= 0 ? 0u : rows <= whole ? 1u : (uint32_t)((rows + slice - 1) / slice);
+    if (rows > whole) atomicAdd(&meta[0], 1ull);
 }
 
 __global__ __launch_bounds__(256) void units_fill_kernel(const int64_t* __restrict__ offs, int64_t P, int64_t slice,
@@ -161,8 +162,8 @@ constexpr int64_t kUnitsSmall = 512;
 
 template <int KB>
 __global__ __launch_bounds__(1024) void units_small_kernel(const void* __restrict__ keys, int64_t n, uint32_t mask,
-                                                           int64_t P, int64_t slice, agg::Unit* __restrict__ units,
-                                                           unsigned long long* meta)
+                                                           int64_t P, int64_t whole, int64_t slice,
+                                                           agg::Unit* __restrict__ units, unsigned long long* meta)
 {
     __shared__ uint32_t wsum[16];
     __shared__ int64_t first[kUnitsSmall + 1];
@@ -196,8 +197,8 @@ __global__ __launch_bounds__(1024) void units_small_kernel(const void* __restric
         cnt[i] = 0;
         if (i < per && (int64_t)t * per + i < P) {
             const int64_t rows = first[t * per + i + 1] - first[t * per + i];
-            cnt[i] = rows <= 0 ? 0u : rows <= slice ? 1u : (uint32_t)((rows + slice - 1) / slice);
-            sliced += rows > slice ? 1u : 0u;
+            cnt[i] = rows <= 0 ? 0u : rows <= whole ? 1u : (uint32_t)((rows + slice - 1) / slice);
+            sliced += rows > whole ? 1u : 0u;
         }
         sum += cnt[i];
     }
@@ -391,14 +392,24 @@ Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream
     std::unique_ptr<HostPhase> phase_units(new HostPhase("host_partition_units", s));
     // Rows per unit: a partition is split when it is much larger than the
     // average (skew), or when there are too few partitions to occupy every CU
-    // twice, since a split partition's groups merge through the HBM table with
-    // atomics instead of being written straight out.  (Splitting at
-    // n / (4 CUs) also with 1024 partitions cut a quarter of them in two: 25M
-    // rows in 700k groups, unit kernel and compaction 289 + 64 us.)
+    // several times, since a split partition's groups merge through the HBM
+    // table with atomics instead of being written straight out.
     const int64_t avg_rows = (n + P - 1) / P;
-    const int64_t balance = std::max<int64_t>(1, n / (4 * (int64_t)di.num_cus));
-    const int64_t fair = P >= 2 * (int64_t)di.num_cus ? 4 * avg_rows : std::min(4 * avg_rows, balance);
-    const int64_t slice = std::max<int64_t>({(int64_t)tune.block * 16, 8 * per_part, fair});
+    const int64_t cus = di.num_cus;
+    const int64_t balance = std::max<int64_t>(1, n / (4 * cus));
+    const int64_t slice = std::max<int64_t>({(int64_t)tune.block * 16, 8 * per_part, std::min(4 * avg_rows, balance)});
+    // From two partitions per CU on, the ones of about the average size stay
+    // whole (2^26 rows in 2^20 groups, 512 partitions, two states: 1466 us with
+    // all of them split, 1245 so).  With fewer than four per CU the last ones
+    // to finish then cost time that grows with the rows, the merges time that
+    // grows with the groups: whole only where the merges cost more (512
+    // partitions, five states, 2^19 groups at Zipf 0.8, split / whole: 2^28
+    // rows 5.55 / 6.08 ms, 2^27 3.03 / 3.21, uniform 2.96 / 2.89, 2^26 1.70 /
+    // 1.70, uniform 1.66 / 1.53, 2^25 1.02 / 0.96).  Larger ones are split
+    // however few they are (whole up to four times the average, 2^28 rows, 2^19
+    // groups at Zipf 1.0: unit kernel 1.6 -> 4.2 ms).
+    const bool whole_avg = P >= 4 * cus || (P >= 2 * cus && 2 * bound * nops > n / 36);
+    const int64_t whole = whole_avg ? std::max(slice, avg_rows + avg_rows / 4) : slice;
     // units built on the device; 16 bytes (unit and sliced-partition counts)
     // come back instead of the boundaries, and no unit list goes up
     const int64_t max_units = P + n / slice + 1;
@@ -414,7 +425,8 @@ Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream
         if (P <= kUnitsSmall) {
             KernelTimer timer("partition_bounds", s);
             auto kern = kb == 4 ? units_small_kernel<4> : units_small_kernel<8>;
-            hipLaunchKernelGGL(kern, dim3(1), dim3(1024), 0, s, pkeys, n, pmask, P, slice, dunits.get<Unit>(), umeta);
+            hipLaunchKernelGGL(kern, dim3(1), dim3(1024), 0, s, pkeys, n, pmask, P, whole, slice, dunits.get<Unit>(),
+                               umeta);
             EG_LAUNCH_CHECK();
         } else {
             offs = DevBuf((size_t)(P + 1) * 8, s);
@@ -428,7 +440,7 @@ Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream
             fill_zero(umeta, 16, s);
             const unsigned ugrid = (unsigned)((P + 255) / 256);
             hipLaunchKernelGGL(units_count_kernel, dim3(ugrid), dim3(256), 0, s, (const int64_t*)offs.get<int64_t>(), P,
-                               slice, cnt, umeta);
+                               whole, slice, cnt, umeta);
             EG_LAUNCH_CHECK();
             scan_exclusive_u32(cnt, pre, P, s, false);
             hipLaunchKernelGGL(units_fill_kernel, dim3(ugrid), dim3(256), 0, s, (const int64_t*)offs.get<int64_t>(), P,

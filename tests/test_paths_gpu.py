@@ -210,3 +210,20 @@ def test_partition_counts_around_the_one_launch_unit_list(bound):
     exp = sorted_by_key(O.groupby(keys, [vals], reqs))
     for fn in (G.partition_groupby, G.partition_groupby_gfur):
         assert_same(sorted_by_key(run(fn, keys, [vals], reqs, G.groupby_hint(groups_upper_bound=min(bound, n - 1)))), exp)
+
+
+@pytest.mark.parametrize("n,bound", [(9_000_011, 500_000), (18_000_011, 800_000), (9_000_011, 300_000)])
+@pytest.mark.parametrize("hot", [0.0, 0.0005, 0.005, 0.3])
+def test_partitions_a_little_larger_than_the_average(n, bound, hot):
+    """512, 1024 and 256 partitions with one from about the average size to
+    many times it: whole below 5/4 of the average, sliced above, or all sliced
+    (256).  The slices' groups come out once and the spill table is used."""
+    rng = np.random.default_rng(bound)
+    keys = O.gen_keys_uniform(n, 20_011, seed=bound)
+    keys[rng.random(n) < hot] = 77
+    vals = O.gen_values(n, O.VAL_UNIFORM_I64, np.int64, seed=4, stream_id=2)
+    reqs = [(0, A.SUM), (0, A.MIN), (0, A.MAX), (-1, A.COUNT_ALL), (0, A.ANY)]
+    exp = sorted_by_key(O.groupby(keys, [vals], reqs[:4]))
+    got = sorted_by_key(run(G.partition_groupby, keys, [vals], reqs, G.groupby_hint(groups_upper_bound=bound)))
+    assert_same(got[:5], exp)
+    assert (exp[2] <= got[5]).all() and (got[5] <= exp[3]).all()
