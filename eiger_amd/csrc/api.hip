@@ -24,9 +24,11 @@ int timing_reset();
 void timing_query(const char* name, int64_t* launches, double* total_ms);
 void zipf_cdf(double* cdf, int64_t distinct, double s);
 Result run_sort(const Plan& plan, const eg_groupby_hint& hint, bool gfur, hipStream_t s);
-Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream_t s);
-// Its radix passes at this bound, and the rows an average partition has.
-int partition_passes(const Plan& plan, int64_t group_bound, int64_t* rows_per_part);
+// expected: about how many groups there are, where more is known than the bound
+// (else the bound).
+Result run_partition(const Plan& plan, int64_t group_bound, int64_t expected, bool gfur, hipStream_t s);
+// Its radix passes, and the rows an average partition has.
+int partition_passes(const Plan& plan, int64_t group_bound, int64_t expected, int64_t* rows_per_part);
 bool mlp_select(const void* keys, int32_t key_type, int64_t rows, int64_t group_bound, int nops, int value_bytes,
                 hipStream_t s, int32_t* algo, int64_t* card_est, float* singletons);
 int64_t ndv_approx(const void* data, int32_t type, int64_t n, hipStream_t s);
@@ -407,6 +409,7 @@ int groupby_entry(Entry entry, const eg_column_view* keys, int64_t num_keys,
 
         int algo;
         int64_t learned_bound = 0;  // group bound from the dispatch model's estimate
+        int64_t expected = 0;       // the estimate itself
         switch (entry) {
         case Entry::HASH: algo = EG_ALGO_HASH; break;
         case Entry::SORT: algo = EG_ALGO_SORT; break;
@@ -451,16 +454,20 @@ int groupby_entry(Entry entry, const eg_column_view* keys, int64_t num_keys,
                     const bool known = h.groups_upper_bound > 0 && h.groups_upper_bound < plan.rows;
                     const int64_t caller = known ? h.groups_upper_bound : plan.rows;
                     learned_bound = std::min<int64_t>(caller, card + card + card / 2 + 1024);
+                    expected = card;
                     int64_t part_rows = 0;
-                    const int passes = known && a == EG_ALGO_PARTITION ? partition_passes(plan, caller, &part_rows) : 0;
+                    const int passes = known && a == EG_ALGO_PARTITION ? partition_passes(plan, caller, card, &part_rows)
+                                                                        : 0;
                     if (plan.rows >= ((int64_t)1 << 24) && passes > 0 &&
-                        passes == partition_passes(plan, learned_bound, nullptr) &&
+                        passes == partition_passes(plan, learned_bound, card, nullptr) &&
                         (passes == 1 || (4 * learned_bound >= caller && part_rows >= 16384))) {
+                        expected = learned_bound;
                         learned_bound = caller;
                     } else if ((learned_bound < caller || !known) && singletons > 0.25f &&
                                plan.rows >= ((int64_t)1 << 24)) {
                         const int64_t est = ndv_approx(plan.key.data, plan.key_type, plan.rows, s);
                         learned_bound = std::min<int64_t>(caller, est + est / 4 + 1024);
+                        expected = est;
                     }
                 } else {
                     int rc = eg_auto_select_algo(kviews, num_keys, &h, stream);
@@ -484,9 +491,12 @@ int groupby_entry(Entry entry, const eg_column_view* keys, int64_t num_keys,
             case EG_ALGO_SORT: case EG_ALGO_SORT_OPT: res = run_sort(plan, h, false, s); break;
             case EG_ALGO_SORT_GFUR: res = run_sort(plan, h, true, s); break;
             case EG_ALGO_PARTITION:
-                res = run_partition(plan, learned_bound > 0 ? learned_bound : group_bound_of(plan, h, s), false, s);
+            case EG_ALGO_PARTITION_GFUR: {
+                const bool learned = learned_bound > 0;
+                const int64_t bound = learned ? learned_bound : group_bound_of(plan, h, s);
+                res = run_partition(plan, bound, learned ? expected : bound, algo == EG_ALGO_PARTITION_GFUR, s);
                 break;
-            case EG_ALGO_PARTITION_GFUR: res = run_partition(plan, group_bound_of(plan, h, s), true, s); break;
+            }
             default: raise(EG_ERR_UNSUPPORTED, "Unsupported groupby algorithm");
             }
         }

@@ -266,9 +266,19 @@ struct PartGeometry {
     int bits;          // log2 partitions
 };
 
-PartGeometry part_geometry(int nops, int kb, int64_t bound)
+// Rows a unit of a sliced partition takes (see run_partition).
+int64_t slice_rows(const PartGeometry& g, int64_t n, int64_t P)
+{
+    const int64_t balance = std::max<int64_t>(1, n / (4 * (int64_t)device_info().num_cus));
+    return std::max<int64_t>({(int64_t)g.tune.block * 16, 8 * g.per_part, std::min(4 * ((n + P - 1) / P), balance)});
+}
+
+// bound: no more groups than that; expected: about how many there are.
+PartGeometry part_geometry(const Plan& plan, int64_t bound, int64_t expected)
 {
     const DeviceInfo& di = device_info();
+    const int nops = plan.spec.nops, kb = plan.key.bytes;
+    const int64_t n = plan.rows;
     PartGeometry g;
     g.tune = part_tune();
     const size_t static_lds = 256;
@@ -283,26 +293,40 @@ PartGeometry part_geometry(int nops, int kb, int64_t bound)
     g.lds = lds_of(g.cr);
     g.per_part = std::max<int64_t>(1, (int64_t)g.cr * 2 / 3);
     g.bits = std::min(24, std::max(1, ceil_log2((bound + g.per_part - 1) / g.per_part)));
-    // Fewer radix passes where the tables then fill to 7/8 of the bound at
-    // most (the bound is an upper one, and an estimate's carries headroom):
-    // 3M rows with a bound of 600k groups take one 8-bit pass instead of two.
+    // Fewer radix passes where the tables then fill to 7/8 of the bound and to
+    // 11/16 of the expected groups at most: an estimate's bound carries
+    // headroom, and 3M rows expected in 200k groups, 500k the bound, take one
+    // 8-bit pass instead of two (264 -> 220 us).  Fuller tables cost far more
+    // than the pass saves: 2^28 rows, five states, 256 partitions against 512
+    // 4.7 / 5.1 ms at 0.68, 5.7 / 5.1 at 0.76, 8.0 / 5.3 at 0.87.  Where the
+    // fewer partitions have to be sliced, their merges (an atomic per state,
+    // group and slice) may not cost more than the pass either: two states,
+    // 561k groups, 2^24 rows 602 / 526 us, 2^26 rows 1155 / 1336.  The two are
+    // even near an atomic per four rows of 16 bytes and per eight of 12.
     const int digit_bits = max_digit_bits();
     const int fewer = (g.bits + digit_bits - 1) / digit_bits * digit_bits - digit_bits;
-    if (fewer >= digit_bits && (bound >> fewer) <= (int64_t)g.cr * 7 / 8) g.bits = fewer;
+    if (fewer >= digit_bits && (bound >> fewer) <= (int64_t)g.cr * 7 / 8 &&
+        (expected >> fewer) <= (int64_t)g.cr * 11 / 16) {
+        int64_t row_bytes = kb;
+        for (int c = 0; c < plan.spec.nvcols; ++c) row_bytes += plan.spec.cols[c].bytes;
+        const int64_t avg = n >> fewer, slice = slice_rows(g, n, (int64_t)1 << fewer);
+        const int64_t slices = (avg + slice - 1) / slice;
+        if (slices <= 1 || expected * nops * slices <= n * std::max<int64_t>(row_bytes - 8, 4) / 32) g.bits = fewer;
+    }
     return g;
 }
 
 }  // namespace
 
-int partition_passes(const Plan& plan, int64_t group_bound, int64_t* rows_per_part)
+int partition_passes(const Plan& plan, int64_t group_bound, int64_t expected, int64_t* rows_per_part)
 {
     const int64_t bound = std::max<int64_t>(1, std::min<int64_t>(group_bound, plan.rows));
-    const int bits = part_geometry(plan.spec.nops, plan.key.bytes, bound).bits;
+    const int bits = part_geometry(plan, bound, std::min(bound, expected)).bits;
     if (rows_per_part) *rows_per_part = plan.rows >> bits;
     return (bits + max_digit_bits() - 1) / max_digit_bits();
 }
 
-Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream_t s)
+Result run_partition(const Plan& plan, int64_t group_bound, int64_t expected, bool gfur, hipStream_t s)
 {
     const DeviceInfo& di = device_info();
     const int64_t n = plan.rows;
@@ -310,7 +334,7 @@ Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream
     const int nops = plan.spec.nops;
     const int64_t bound = std::max<int64_t>(1, std::min<int64_t>(group_bound, n));
 
-    const PartGeometry geo = part_geometry(nops, kb, bound);
+    const PartGeometry geo = part_geometry(plan, bound, std::min(bound, expected));
     const PartTune tune = geo.tune;
     const int cr = geo.cr, bits = geo.bits;
     const size_t lds = geo.lds;
@@ -396,8 +420,7 @@ Result run_partition(const Plan& plan, int64_t group_bound, bool gfur, hipStream
     // table with atomics instead of being written straight out.
     const int64_t avg_rows = (n + P - 1) / P;
     const int64_t cus = di.num_cus;
-    const int64_t balance = std::max<int64_t>(1, n / (4 * cus));
-    const int64_t slice = std::max<int64_t>({(int64_t)tune.block * 16, 8 * per_part, std::min(4 * avg_rows, balance)});
+    const int64_t slice = slice_rows(geo, n, P);
     // From two partitions per CU on, the ones of about the average size stay
     // whole (2^26 rows in 2^20 groups, 512 partitions, two states: 1466 us with
     // all of them split, 1245 so).  With fewer than four per CU the last ones

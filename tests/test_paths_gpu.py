@@ -227,3 +227,38 @@ def test_partitions_a_little_larger_than_the_average(n, bound, hot):
     got = sorted_by_key(run(G.partition_groupby, keys, [vals], reqs, G.groupby_hint(groups_upper_bound=bound)))
     assert_same(got[:5], exp)
     assert (exp[2] <= got[5]).all() and (got[5] <= exp[3]).all()
+
+
+@pytest.mark.parametrize("states,slots", [(2, 4060), (3, 2912), (12, 800)])
+@pytest.mark.parametrize("fill,passes", [(0.5, 1), (0.65, 1), (0.8, 2), (0.87, 2)])
+def test_partition_passes_at_a_true_bound(states, slots, fill, passes):
+    """256 tables of about `slots` slots as full as the bound says: one digit
+    pass up to 2/3 full, above that two passes into more partitions."""
+    n, d = 1_500_007, int(256 * slots * fill)
+    _check_partitioned(n, d, d, states, passes)
+
+
+@pytest.mark.parametrize("states,slots", [(2, 4060), (3, 2912), (12, 800)])
+@pytest.mark.parametrize("fill", [0.85, 0.95, 1.1])
+def test_partition_tables_fuller_than_planned(states, slots, fill):
+    """More groups than the bound: the unit tables fill to `fill` of their
+    slots, keys whose buckets are full go to the HBM table (and where that
+    fills too, the call runs again with a larger one)."""
+    _check_partitioned(1_500_007, int(256 * slots * fill), int(256 * slots * 0.6), states, 1)
+
+
+def _check_partitioned(n, d, bound, states, passes):
+    rng = np.random.default_rng(d)
+    keys = np.concatenate([rng.permutation(d), rng.integers(0, d, n - d)]).astype(np.int32)
+    vals = [rng.integers(-1000, 1000, n).astype(np.int64) for _ in range(4)]
+    reqs = ([(-1, A.COUNT_ALL)] + [(c, k) for k in (A.SUM, A.MIN, A.MAX) for c in range(4)])[:states]
+    exp = sorted_by_key(O.groupby(keys, vals, reqs))
+    try:
+        G.kernel_timing(True)
+        G.kernel_timing_reset()
+        got = sorted_by_key(run(G.partition_groupby, keys, vals, reqs, G.groupby_hint(groups_upper_bound=bound)))
+        assert G.kernel_time("radix_scatter")[0] == passes
+    finally:
+        G.kernel_timing(False)
+        G.kernel_timing_reset()
+    assert_same(got, exp)
