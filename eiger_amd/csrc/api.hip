@@ -24,11 +24,6 @@ int timing_reset();
 void timing_query(const char* name, int64_t* launches, double* total_ms);
 void zipf_cdf(double* cdf, int64_t distinct, double s);
 Result run_sort(const Plan& plan, const eg_groupby_hint& hint, bool gfur, hipStream_t s);
-// expected: about how many groups there are, where more is known than the bound
-// (else the bound).
-Result run_partition(const Plan& plan, int64_t group_bound, int64_t expected, bool gfur, hipStream_t s);
-// Its radix passes, and the rows an average partition has.
-int partition_passes(const Plan& plan, int64_t group_bound, int64_t expected, int64_t* rows_per_part);
 bool mlp_select(const void* keys, int32_t key_type, int64_t rows, int64_t group_bound, int nops, int value_bytes,
                 hipStream_t s, int32_t* algo, int64_t* card_est, float* singletons);
 int64_t ndv_approx(const void* data, int32_t type, int64_t n, hipStream_t s);
@@ -309,6 +304,56 @@ Result wide_groupby(const ViewIn& k, const std::vector<ViewIn>& vs, const eg_agg
     return all;
 }
 
+// Sizing of a dispatched call's tables.
+struct GroupSizing {
+    int64_t caller;      // the caller's bound, or the rows
+    int64_t bound;       // no more groups than that
+    int64_t expected;    // about how many
+    bool full_estimate;  // replace both by the full-column HyperLogLog estimate
+};
+
+// The tables are sized from a group-count bound.  A caller's bound is an upper
+// bound, often loose (skewed keys use few of the possible values), so a
+// smaller estimate replaces it: the model's estimate with 2.5x headroom.  On
+// inputs of 2^24 rows or more whose sample is mostly singletons (more than 1/4
+// of its keys seen once) the model's estimate can be too low by more than the
+// headroom (up to 3.3x over 2^24 to 2^28 rows in 2^11 to 2^26 keys), and the
+// full-column HyperLogLog estimate (standard error 0.8%, 25% headroom) sizes
+// the tables instead: one pass over the keys (0.25 ms per 2^28 rows and a
+// synchronisation), cheap against such an input, and tighter tables.
+// - With no caller bound it runs whatever the estimate (67M rows in 16.7M
+//   groups were cut into 32768 partitions for the row count as bound: 2.98 ->
+//   2.75 ms).
+// - With one, and the partition strategy, only where the tighter bound saves
+//   enough: a radix pass; digit bits, where rows times bits reach 2^27 (2^28
+//   rows with 2^18 as bound, in 2^13 groups 4.3 ms without the estimate, 3.5
+//   with it, in 2^16 groups, which saves no bit, 3.86 / 3.75; 2^24 rows in 2^13
+//   groups 0.46 / 0.57), of one pass of less than 8 bits 2^29 (2^28 rows, 2^17 as
+//   bound for 2^15 groups 3.92 / 4.19); or where the partitions of two passes
+//   are so small (16384 rows) that fewer of them make a faster unit kernel
+//   (2^28 rows, Zipf 1.0, 2^26 as bound for 30M groups: 8.0 ms without, 7.4
+//   with).  Else the caller's bound stands.
+// Below 2^24 rows the pass and its synchronisation would cost more than the
+// tighter sizing saves; the model's estimate stays within 1.34x of the true
+// count on every held-out query of that kind (2,913), far inside the headroom.
+GroupSizing dispatch_sizing(const Plan& plan, int algo, int64_t group_bound, int64_t card, float singletons)
+{
+    const bool known = group_bound > 0 && group_bound < plan.rows;
+    GroupSizing z{known ? group_bound : plan.rows, 0, card, false};
+    z.bound = std::min<int64_t>(z.caller, card + card + card / 2 + 1024);
+    z.full_estimate = plan.rows >= ((int64_t)1 << 24) && singletons > 0.25f && (z.bound < z.caller || !known);
+    if (!z.full_estimate || !known || algo != EG_ALGO_PARTITION) return z;
+    const PartitionShape loose = partition_shape(plan, z.caller, z.bound), tight = partition_shape(plan, z.bound, card);
+    const int64_t worth = (int64_t)1 << (loose.bits < 8 ? 29 : 27);
+    z.full_estimate = loose.passes != tight.passes || (loose.bits - tight.bits) * plan.rows >= worth ||
+                      (loose.passes > 1 && loose.part_rows < 16384);
+    if (!z.full_estimate) {
+        z.expected = z.bound;
+        z.bound = z.caller;
+    }
+    return z;
+}
+
 int groupby_entry(Entry entry, const eg_column_view* keys, int64_t num_keys,
                   const eg_column_view* vals, int64_t num_vals, const eg_agg_request* reqs,
                   int64_t num_reqs, eg_groupby_hint* hint, void* stream, eg_table* out)
@@ -427,46 +472,12 @@ int groupby_entry(Entry entry, const eg_column_view* keys, int64_t num_keys,
                 if (mlp_select(plan.key.data, plan.key_type, plan.rows, h.groups_upper_bound, plan.spec.nops, vbytes, s,
                                &a, &card, &singletons)) {
                     h.groupby_algo = a;
-                    // The tables are sized from a group-count bound.  A caller's
-                    // bound is an upper bound, often loose (skewed keys use few
-                    // of the possible values), so a smaller estimate replaces
-                    // it: the model's estimate with 2.5x headroom.  On inputs
-                    // of 2^24 rows or more whose sample is mostly singletons
-                    // (more than 1/4 of its keys seen once) the full-column
-                    // HyperLogLog estimate (standard error 0.8%, 25% headroom)
-                    // sizes the tables instead: one pass over the keys, cheap
-                    // against such an input, and tighter tables.  With no
-                    // caller bound it runs whatever the estimate (67M rows in
-                    // 16.7M groups were cut into 32768 partitions for the row
-                    // count as bound: 2.98 -> 2.75 ms).  With one, and the
-                    // partition strategy, only where a tighter bound could
-                    // save a radix pass, two digit bits of two passes, or
-                    // where the partitions are so small (16384 rows) that
-                    // fewer of them make a faster unit kernel (2^28 rows, Zipf
-                    // 1.0, 2^26 as bound for 30M groups: 8.0 ms without the
-                    // estimate, 7.4 with it): else it costs more (0.25 ms per
-                    // 2^28 rows) than it saves.
-                    // Below 2^24 rows the pass and its synchronisation would
-                    // cost more than the tighter sizing saves; the model's
-                    // estimate stays within 1.34x of the true count on every
-                    // held-out query of that kind (2,913), far inside the
-                    // headroom.
-                    const bool known = h.groups_upper_bound > 0 && h.groups_upper_bound < plan.rows;
-                    const int64_t caller = known ? h.groups_upper_bound : plan.rows;
-                    learned_bound = std::min<int64_t>(caller, card + card + card / 2 + 1024);
-                    expected = card;
-                    int64_t part_rows = 0;
-                    const int passes = known && a == EG_ALGO_PARTITION ? partition_passes(plan, caller, card, &part_rows)
-                                                                        : 0;
-                    if (plan.rows >= ((int64_t)1 << 24) && passes > 0 &&
-                        passes == partition_passes(plan, learned_bound, card, nullptr) &&
-                        (passes == 1 || (4 * learned_bound >= caller && part_rows >= 16384))) {
-                        expected = learned_bound;
-                        learned_bound = caller;
-                    } else if ((learned_bound < caller || !known) && singletons > 0.25f &&
-                               plan.rows >= ((int64_t)1 << 24)) {
+                    const GroupSizing z = dispatch_sizing(plan, a, h.groups_upper_bound, card, singletons);
+                    learned_bound = z.bound;
+                    expected = z.expected;
+                    if (z.full_estimate) {
                         const int64_t est = ndv_approx(plan.key.data, plan.key_type, plan.rows, s);
-                        learned_bound = std::min<int64_t>(caller, est + est / 4 + 1024);
+                        learned_bound = std::min<int64_t>(z.caller, est + est / 4 + 1024);
                         expected = est;
                     }
                 } else {
@@ -521,6 +532,28 @@ void eg_hint_init(eg_groupby_hint* h)
     h->agg_count = 0;
     h->enable_skf = 0;
     h->allow_hash_fallback = 0;
+}
+
+int eg_dispatch_sizing(int32_t key_type, int64_t rows, int64_t groups_upper_bound, int32_t nops, int32_t value_bytes,
+                       int32_t algo, int64_t card, float singletons, int64_t* bound, int64_t* expected,
+                       int32_t* full_estimate)
+{
+    return guard([&] {
+        if (rows < 0 || nops < 1 || nops > kMaxOps || value_bytes < 0 || !bound || !expected || !full_estimate)
+            raise(EG_ERR_INVALID, "eg_dispatch_sizing: bad arguments");
+        Plan plan;
+        plan.rows = rows;
+        plan.key_type = key_type;
+        plan.key.bytes = type_size(key_type);
+        if (plan.key.bytes != 4 && plan.key.bytes != 8) raise(EG_ERR_UNSUPPORTED, "eg_dispatch_sizing: key type");
+        plan.spec.nops = nops;
+        plan.spec.nvcols = 1;  // the row width is all that counts
+        plan.spec.cols[0].bytes = value_bytes;
+        const GroupSizing z = dispatch_sizing(plan, algo, groups_upper_bound, card, singletons);
+        *bound = z.bound;
+        *expected = z.expected;
+        *full_estimate = z.full_estimate ? 1 : 0;
+    });
 }
 
 int eg_groupby(const eg_column_view* keys, int64_t num_keys, const eg_column_view* vals,

@@ -233,6 +233,18 @@ struct HashTuning {
 
 Result run_hash(const Plan& plan, int64_t group_bound, hipStream_t s, const HashTuning& t = HashTuning{});
 
+// expected: about how many groups there are, where more is known than the bound
+// (else the bound).
+Result run_partition(const Plan& plan, int64_t group_bound, int64_t expected, bool gfur, hipStream_t s);
+
+// How run_partition would cut the rows.
+struct PartitionShape {
+    int bits;           // log2 partitions
+    int passes;         // radix passes
+    int64_t part_rows;  // rows of an average partition
+};
+PartitionShape partition_shape(const Plan& plan, int64_t group_bound, int64_t expected);
+
 // The hash strategy into caller-owned outputs (os, `capacity` rows each) with
 // its HBM table in the library's static device scratch: no device memory is
 // allocated or freed.  Returns the group count; raises EG_ERR_CAPACITY when

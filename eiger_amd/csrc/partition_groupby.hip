@@ -318,12 +318,11 @@ PartGeometry part_geometry(const Plan& plan, int64_t bound, int64_t expected)
 
 }  // namespace
 
-int partition_passes(const Plan& plan, int64_t group_bound, int64_t expected, int64_t* rows_per_part)
+PartitionShape partition_shape(const Plan& plan, int64_t group_bound, int64_t expected)
 {
     const int64_t bound = std::max<int64_t>(1, std::min<int64_t>(group_bound, plan.rows));
     const int bits = part_geometry(plan, bound, std::min(bound, expected)).bits;
-    if (rows_per_part) *rows_per_part = plan.rows >> bits;
-    return (bits + max_digit_bits() - 1) / max_digit_bits();
+    return PartitionShape{bits, (bits + max_digit_bits() - 1) / max_digit_bits(), plan.rows >> bits};
 }
 
 Result run_partition(const Plan& plan, int64_t group_bound, int64_t expected, bool gfur, hipStream_t s)

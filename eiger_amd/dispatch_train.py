@@ -45,7 +45,8 @@ A = G.aggregation_id
 T = G.type_id
 STRATS = ("hash", "sort", "partition")
 FNS = {"hash": G.hash_groupby, "sort": G.sort_groupby, "partition": G.partition_groupby}
-ALGO_INDEX = {G.groupby_algo.HASH: 0, G.groupby_algo.SORT: 1, G.groupby_algo.PARTITION: 2}
+ALGOS = (G.groupby_algo.HASH, G.groupby_algo.SORT, G.groupby_algo.PARTITION)
+ALGO_INDEX = {a: i for i, a in enumerate(ALGOS)}
 REQS_BATCH = [(0, A.SUM), (-1, A.COUNT_ALL)]
 REQS_SWEEP = [(-1, A.COUNT_ALL), (0, A.SUM), (0, A.MIN), (0, A.MAX), (1, A.SUM)]
 
@@ -120,19 +121,18 @@ def trace(specs, seed0: int, wl: Workload, progress_every: int = 500):
         _, rule_ms[i] = timed(G.auto_select_groupby_algo, [k], h)
         rule[i] = ALGO_INDEX.get(h.groupby_algo, 0)
         # the true group count (untimed), then every strategy sized the way the
-        # learned dispatcher sizes the one it picks (api.hip: 2.5x the
-        # estimate, or the HyperLogLog estimate + 25% when the sample is mostly
-        # singletons), with the true count standing in for the estimates
+        # dispatcher sizes the one it picks, with the true count standing in
+        # for the estimates (partition by its own entry, which takes the bound
+        # for the expected count too)
         t = FNS["hash"]([k], vals, reqs, G.groupby_hint(groups_upper_bound=spec[2]))
         true = int(t.num_rows())
         t.free()
         rows = spec[1]
-        caller = spec[2] if 0 < spec[2] < rows else rows
-        bound = min(caller, 2 * true + true // 2 + 1024)
-        if bound < caller and feats[i][7] > 0.25:
-            bound = min(caller, true + true // 4 + 1024)
         groups[i] = true
         for j, name in enumerate(STRATS):
+            bound, _, full = G.dispatch_sizing(T.INT32, rows, spec[2], nops, vb, ALGOS[j], true, feats[i][7])
+            if full:
+                bound = min(spec[2] if 0 < spec[2] < rows else rows, true + true // 4 + 1024)
             hint = G.groupby_hint(groups_upper_bound=bound)
             t, times[i, j] = timed(FNS[name], [k], vals, reqs, hint)
             t.free()

@@ -795,6 +795,17 @@ def mlp_select(key: column_view, group_bound=0, nops=2, value_bytes=8, stream=No
     return groupby_algo(a.value), card.value
 
 
+def dispatch_sizing(key_type: int, rows: int, group_bound: int, nops: int, value_bytes: int, algo: int, card: int,
+                    singletons: float):
+    """(bound, expected groups, full estimate?) that AUTO sizes its tables with
+    for the model's strategy and estimate and its sample's singleton share
+    (mlp_features column 7)."""
+    b, e, f = C.c_int64(), C.c_int64(), C.c_int32()
+    _check(lib().eg_dispatch_sizing(int(key_type), int(rows), int(group_bound), int(nops), int(value_bytes), int(algo),
+                                    int(card), float(singletons), C.byref(b), C.byref(e), C.byref(f)))
+    return b.value, e.value, bool(f.value)
+
+
 def _mlp_queries(keys, group_bounds, nops, value_bytes):
     n = len(keys)
     arr = (_lib_mod.MlpQuery * max(n, 1))()

@@ -409,6 +409,14 @@ int eg_mlp_loaded(void);
  * estimate for one key column. */
 int eg_mlp_select(eg_column_view key, int64_t group_bound, int32_t nops, int32_t value_bytes, void* stream,
                   int32_t* algo, int64_t* card_est);
+/* The group bound that eg_groupby's AUTO sizes its tables with, from the model's
+ * strategy and estimate (eg_mlp_select) and the share of singletons in its
+ * sample (feature 7): *bound, the group count it expects, and whether a
+ * full-column estimate replaces both.  groups_upper_bound: the caller's hint.
+ * Reads and launches nothing. */
+int eg_dispatch_sizing(int32_t key_type, int64_t rows, int64_t groups_upper_bound, int32_t nops, int32_t value_bytes,
+                       int32_t algo, int64_t card, float singletons, int64_t* bound, int64_t* expected,
+                       int32_t* full_estimate);
 /* The loaded model's choice for `num` queries: one feature launch, one
  * forward launch, one synchronisation. */
 int eg_mlp_select_batch(const eg_mlp_query* queries, int64_t num, int32_t* algos, int64_t* card_est,

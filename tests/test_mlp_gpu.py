@@ -127,3 +127,27 @@ def test_batched_selection_equals_single_query_selection():
             assert a1 == a and c1 == c
     finally:
         G.mlp_load(None)
+
+
+@pytest.mark.parametrize("log_rows,bound,algo,card,singles,exp", [
+    # (bound, expected, full estimate): the estimate with headroom, or the caller's bound
+    (20, 1 << 18, "PARTITION", 10_000, 0.9, (26_024, 10_000, False)),
+    (20, 20_000, "PARTITION", 10_000, 0.9, (20_000, 10_000, False)),
+    (24, 1 << 18, "PARTITION", 10_000, 0.2, (26_024, 10_000, False)),     # few singletons: the estimate stands
+    (28, 1 << 24, "PARTITION", 2_000_000, 0.2, (5_001_024, 2_000_000, False)),
+    (24, 1 << 18, "PARTITION", 10_000, 0.9, (1 << 18, 26_024, False)),    # 2^24 rows: three digit bits do not pay
+    (28, 1 << 18, "PARTITION", 10_000, 0.9, (26_024, 10_000, True)),      # 2^28 rows: they do
+    (28, 1 << 18, "PARTITION", 100_000, 0.9, (1 << 18, 251_024, False)),  # no digit bit saved
+    (28, 1 << 17, "PARTITION", 25_000, 0.9, (1 << 17, 63_524, False)),    # seven bits to six
+    (28, 1 << 22, "PARTITION", 50_000, 0.9, (126_024, 50_000, True)),     # a pass saved
+    (28, 1 << 24, "PARTITION", 6_000_000, 0.9, (1 << 24, 15_001_024, False)),
+    (28, 1 << 26, "PARTITION", 20_000_000, 0.9, (50_001_024, 20_000_000, True)),  # small partitions
+    (28, 1 << 18, "HASH", 10_000, 0.9, (26_024, 10_000, True)),
+    (28, 0, "PARTITION", 10_000, 0.9, (26_024, 10_000, True)),            # no caller bound
+    (24, 0, "PARTITION", 1 << 24, 0.9, (1 << 24, 1 << 24, True)),
+])
+def test_sizing_of_dispatched_tables(log_rows, bound, algo, card, singles, exp):
+    """Five states over rows of 16 bytes: each side of the lines between the
+    model's estimate, the caller's bound and the full-column estimate."""
+    got = G.dispatch_sizing(G.type_id.INT32, 1 << log_rows, bound, 5, 12, G.groupby_algo[algo], card, singles)
+    assert got == exp
