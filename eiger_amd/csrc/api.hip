@@ -453,8 +453,8 @@ int groupby_entry(Entry entry, const eg_column_view* keys, int64_t num_keys,
         plan.key.data = k.data;
 
         int algo;
-        int64_t learned_bound = 0;  // group bound from the dispatch model's estimate
-        int64_t expected = 0;       // the estimate itself
+        int64_t group_bound = 0;  // from the dispatch model's estimate, else from the hint
+        int64_t expected = 0;     // the estimate itself, else the bound
         switch (entry) {
         case Entry::HASH: algo = EG_ALGO_HASH; break;
         case Entry::SORT: algo = EG_ALGO_SORT; break;
@@ -473,11 +473,11 @@ int groupby_entry(Entry entry, const eg_column_view* keys, int64_t num_keys,
                                &a, &card, &singletons)) {
                     h.groupby_algo = a;
                     const GroupSizing z = dispatch_sizing(plan, a, h.groups_upper_bound, card, singletons);
-                    learned_bound = z.bound;
+                    group_bound = z.bound;
                     expected = z.expected;
                     if (z.full_estimate) {
                         const int64_t est = ndv_approx(plan.key.data, plan.key_type, plan.rows, s);
-                        learned_bound = std::min<int64_t>(z.caller, est + est / 4 + 1024);
+                        group_bound = std::min<int64_t>(z.caller, est + est / 4 + 1024);
                         expected = est;
                     }
                 } else {
@@ -497,17 +497,15 @@ int groupby_entry(Entry entry, const eg_column_view* keys, int64_t num_keys,
             OutSpec os;
             alloc_outputs(plan, 0, s, res, os);
         } else {
+            if (algo == EG_ALGO_HASH || algo == EG_ALGO_PARTITION || algo == EG_ALGO_PARTITION_GFUR) {
+                if (group_bound == 0) group_bound = expected = group_bound_of(plan, h, s);
+            }
             switch (algo) {
-            case EG_ALGO_HASH: res = run_hash(plan, learned_bound > 0 ? learned_bound : group_bound_of(plan, h, s), s); break;
+            case EG_ALGO_HASH: res = run_hash(plan, group_bound, expected, s); break;
             case EG_ALGO_SORT: case EG_ALGO_SORT_OPT: res = run_sort(plan, h, false, s); break;
             case EG_ALGO_SORT_GFUR: res = run_sort(plan, h, true, s); break;
-            case EG_ALGO_PARTITION:
-            case EG_ALGO_PARTITION_GFUR: {
-                const bool learned = learned_bound > 0;
-                const int64_t bound = learned ? learned_bound : group_bound_of(plan, h, s);
-                res = run_partition(plan, bound, learned ? expected : bound, algo == EG_ALGO_PARTITION_GFUR, s);
-                break;
-            }
+            case EG_ALGO_PARTITION: res = run_partition(plan, group_bound, expected, false, s); break;
+            case EG_ALGO_PARTITION_GFUR: res = run_partition(plan, group_bound, expected, true, s); break;
             default: raise(EG_ERR_UNSUPPORTED, "Unsupported groupby algorithm");
             }
         }

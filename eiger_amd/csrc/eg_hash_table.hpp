@@ -132,7 +132,8 @@ struct HashLayout {
     int peel_min = 8;
 };
 
-HashLayout plan_hash_layout(int nops, int key_bytes, int64_t group_bound, const HashTuning& t);
+// expected: about how many groups there are (at most the bound).
+HashLayout plan_hash_layout(int nops, int key_bytes, int64_t group_bound, int64_t expected, const HashTuning& t);
 #endif
 
 }  // namespace eg

@@ -231,10 +231,11 @@ struct HashTuning {
     int64_t table_slots = 0;  // 0 = from the group bound
 };
 
-Result run_hash(const Plan& plan, int64_t group_bound, hipStream_t s, const HashTuning& t = HashTuning{});
-
 // expected: about how many groups there are, where more is known than the bound
 // (else the bound).
+Result run_hash(const Plan& plan, int64_t group_bound, int64_t expected, hipStream_t s, const HashTuning& t = HashTuning{});
+
+// expected: as run_hash's.
 Result run_partition(const Plan& plan, int64_t group_bound, int64_t expected, bool gfur, hipStream_t s);
 
 // How run_partition would cut the rows.
@@ -244,6 +245,9 @@ struct PartitionShape {
     int64_t part_rows;  // rows of an average partition
 };
 PartitionShape partition_shape(const Plan& plan, int64_t group_bound, int64_t expected);
+
+// Slots of a workgroup's LDS table in the hash strategy (one replica).
+int hash_lds_slots(int nops, int key_bytes);
 
 // The hash strategy into caller-owned outputs (os, `capacity` rows each) with
 // its HBM table in the library's static device scratch: no device memory is

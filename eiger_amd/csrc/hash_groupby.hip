@@ -33,6 +33,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <mutex>
 #include <type_traits>
@@ -93,12 +94,14 @@ void launch_compact(const GTable& gt, const OutSpec& os, unsigned long long* cou
 // one.  Measured on both sides, two and five states, us flushed / stored:
 // 2^16 rows, 200 groups 45/48, 400 54/50; 2^18, 64 47/48, 128 51/49;
 // 2^20, 16 52/49, 1000 306/60; 2^26, 64 248/244, 128 274/246; 2^28 (five
-// states), 16 766/832, 200 789/796, 400 891/808.
-bool store_pays(int64_t rows, int64_t bound)
+// states), 16 766/832, 200 789/796, 400 891/808.  Above two value columns a
+// block has half the threads: 2^26 rows, 12 states, 100 groups 1025/1100.
+bool store_pays(int64_t rows, int64_t groups, int nvcols)
 {
-    const int64_t tiles = (rows + 4095) / 4096;
+    const int64_t tile = nvcols <= 2 ? 4096 : 2048;
+    const int64_t tiles = (rows + tile - 1) / tile;
     const int64_t blocks = std::min<int64_t>(tiles, device_info().num_cus);
-    return blocks * bound >= 6400 + tiles;
+    return blocks * groups >= 5000 + tiles;
 }
 
 // The aggregation of n rows into gt.  `scratch` (optional): where the blocks'
@@ -138,7 +141,7 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 }  // namespace
 
-HashLayout plan_hash_layout(int nops, int key_bytes, int64_t group_bound, const HashTuning& t)
+HashLayout plan_hash_layout(int nops, int key_bytes, int64_t group_bound, int64_t expected, const HashTuning& t)
 {
     const DeviceInfo& di = device_info();
     HashLayout L;
@@ -178,9 +181,18 @@ HashLayout plan_hash_layout(int nops, int key_bytes, int64_t group_bound, const 
     // A table much smaller than the group count still catches the hot keys
     // (they arrive early); keep the probing short so cold rows spill cheaply.
     const int64_t slots = std::max(L.cr, 1);
-    L.probe_limit = group_bound > 4 * slots ? 2 : group_bound > slots ? 4 : 16;
+    L.probe_limit = expected > 4 * slots ? 2 : expected > slots ? 4 : 16;
     L.peel_min = t.peel_min;
     return L;
+}
+
+int hash_lds_slots(int nops, int key_bytes)
+{
+    static std::atomic<int> known[2][kMaxOps + 1];  // the same on every device of one architecture
+    nops = std::min(std::max(nops, 1), kMaxOps);
+    std::atomic<int>& slots = known[key_bytes == 8 ? 1 : 0][nops];
+    if (slots == 0) slots = plan_hash_layout(nops, key_bytes, (int64_t)1 << 30, 0, HashTuning{}).cr;
+    return slots;
 }
 
 // ---- tiny inputs ---------------------------------------------------------------
@@ -294,7 +306,7 @@ bool run_tiny(const Plan& plan, const HashTuning& t, hipStream_t s, Result& res)
 // the group count (at most 40 bytes a group for the benchmark's requests).
 constexpr int64_t kEarlyOutputRows = (int64_t)1 << 22;
 
-Result run_hash(const Plan& plan, int64_t group_bound, hipStream_t s, const HashTuning& t)
+Result run_hash(const Plan& plan, int64_t group_bound, int64_t expected, hipStream_t s, const HashTuning& t)
 {
     const int64_t n = plan.rows;
     const int nops = plan.spec.nops;
@@ -304,12 +316,13 @@ Result run_hash(const Plan& plan, int64_t group_bound, hipStream_t s, const Hash
         Result res;
         if (KB == 4 ? run_tiny<4>(plan, t, s, res) : run_tiny<8>(plan, t, s, res)) return res;
     }
-    const HashLayout L = plan_hash_layout(nops, KB, group_bound, t);
+    const HashLayout L = plan_hash_layout(nops, KB, group_bound, std::min(group_bound, expected), t);
 
     bool vec = aligned16(plan.key.data);
     for (int c = 0; c < plan.spec.nvcols; ++c) vec = vec && aligned16(plan.spec.cols[c].data);
 
     int64_t bound = std::max<int64_t>(1, std::min<int64_t>(group_bound, n));
+    expected = std::max<int64_t>(1, std::min(expected, bound));
     int64_t slots = t.table_slots > 0 ? t.table_slots : 1024;
     while (slots < 2 * bound) slots <<= 1;
 
@@ -325,9 +338,9 @@ Result run_hash(const Plan& plan, int64_t group_bound, hipStream_t s, const Hash
         OutSpec eos;
         if (early) alloc_outputs(plan, bound, s, eres, eos);
         DevBuf scratch;
-        // bounds above twice the LDS slots flush: the tables then hold different
-        // keys (3M rows in 400k groups 329 us flushed, 622 stored and merged)
-        DevBuf* stored = bound <= 2 * (int64_t)L.cr && store_pays(n, bound) ? &scratch : nullptr;
+        // above twice the LDS slots the tables hold different keys and flush (3M
+        // rows in 400k groups 329 us, 622 stored and merged)
+        DevBuf* stored = expected <= 2 * (int64_t)L.cr && store_pays(n, expected, plan.spec.nvcols) ? &scratch : nullptr;
         if (KB == 4) aggregate<4>(vec, t, plan.key, n, plan.spec, ht.gt, L, s, true, stored);
         else aggregate<8>(vec, t, plan.key, n, plan.spec, ht.gt, L, s, true, stored);
         if (early) launch_compact(ht.gt, eos, ht.gt.meta + 3, s, bound);  // meta[3]: zeroed with the table
@@ -396,7 +409,7 @@ int64_t run_hash_noalloc(const Plan& plan, int64_t group_bound, const OutSpec& o
     const int W = table_words_per_slot(nops);
     const int KB = plan.key.bytes;
     const HashTuning t;
-    const HashLayout L = plan_hash_layout(nops, KB, group_bound, t);
+    const HashLayout L = plan_hash_layout(nops, KB, group_bound, group_bound, t);
     bool vec = aligned16(plan.key.data);
     for (int c = 0; c < plan.spec.nvcols; ++c) vec = vec && aligned16(plan.spec.cols[c].data);
 

@@ -593,31 +593,45 @@ LoadedModel& loaded_model()
 constexpr int64_t kSmallRows = (int64_t)1 << 17;
 
 // Group counts up to which an input goes to hash whatever the class scores:
-// its tables then fit one workgroup's LDS, and a streaming pass with one merge
-// of the workgroups' tables beats radix passes.  2^24 rows and more: the
-// fastest for all such queries of the training and held-out traces (estimate
-// <= 2048).  Below: half of that, which leaves the bound made of an estimate
-// (2.5x) inside the LDS table for up to ten states; 2^20 rows in 1024 groups
-// 62 us by hash, 132 by partition.
-double hash_card(int64_t rows) { return rows >= ((int64_t)1 << 24) ? 2048.0 : 1280.0; }
+// its groups then fit one workgroup's LDS table, and a streaming pass with one
+// merge of the workgroups' tables beats radix passes.  2048 (the fastest for
+// all such queries of the training and held-out traces with 2^24 rows or more),
+// and within the table's slots, which are fewer with more states (ten: 1936; 16:
+// 1200).  us by hash / partition: 2^17 rows, two states, 1280 groups 66 / 107; 2^20
+// rows, 1280 groups 80 / 110, ten states, 1000 groups 100 / 179; 2^22 rows, eight
+// states, 2000 groups 209 / 311; 2^26 rows, eight states, 1600 groups 640 / 1150.
+// A caller's bound, which is seldom reached, may exceed the slots: up to 1280
+// (2^20 rows, 16 states, 1250 groups 144 / 199), with 2^24 rows or more to 2048.
+constexpr int64_t kHashGroups = 2048;
+
+double hash_card(int nops, int key_bytes) { return (double)std::min<int64_t>(kHashGroups, hash_lds_slots(nops, key_bytes)); }
 
 // Strategy from the model's outputs o[0..3] (class scores of hash / sort /
 // partition, log2 group count / 32), after hash_card's rule.
-int algo_of(const float* o, int64_t rows)
+int algo_of(const float* o, int64_t rows, int nops, int key_bytes)
 {
     if (rows < kSmallRows) return EG_ALGO_HASH;
     const double card = std::exp2(std::min(62.0, std::max(0.0, (double)o[3] * 32.0)));
-    if (card <= hash_card(rows)) return EG_ALGO_HASH;
+    if (card <= hash_card(nops, key_bytes)) return EG_ALGO_HASH;
     const int best = (o[1] > o[0] && o[1] >= o[2]) ? 1 : (o[2] > o[0] && o[2] > o[1]) ? 2 : 0;
     return best == 0 ? EG_ALGO_HASH : best == 1 ? EG_ALGO_SORT : EG_ALGO_PARTITION;
 }
 
 // An input whose caller-given group bound already meets that rule goes to
-// hash without sampling: the bound caps the true group count, so
-// algo_of's rule would pick hash for any estimate the model could give.
-bool bound_picks_hash(int64_t rows, int64_t group_bound)
+// hash without sampling: the bound caps the true group count.
+bool bound_picks_hash(int64_t rows, int64_t group_bound, int nops, int key_bytes)
 {
-    return rows >= kSmallRows && group_bound > 0 && (double)group_bound <= hash_card(rows);
+    if (rows < kSmallRows || group_bound <= 0 || group_bound > kHashGroups) return false;
+    return rows >= ((int64_t)1 << 24) || group_bound <= std::max(1280, hash_lds_slots(nops, key_bytes));
+}
+
+// A query as the model is asked about it.  Its traces have two and five states
+// over 8 and 12 bytes of values; beyond those the group estimate goes astray
+// (0.56 to 1.72 times the true count within; ten states over 32 bytes: 3 for
+// 600 groups, 84 for 4000), so wider requests count as the widest of them.
+FQuery select_query(const void* keys, int64_t rows, int64_t group_bound, int key_bytes, int nops, int value_bytes)
+{
+    return FQuery{keys, rows, group_bound, key_bytes, std::min(nops, 5), std::min(value_bytes, 12), 0};
 }
 
 // Learned strategy choice for one key column; false when no model is loaded.
@@ -627,14 +641,15 @@ bool mlp_select(const void* keys, int32_t key_type, int64_t rows, int64_t group_
     LoadedModel& m = loaded_model();
     std::lock_guard<std::mutex> lk(m.mu);
     if (!m.loaded) return false;
-    if (rows < kSmallRows || bound_picks_hash(rows, group_bound)) {
+    const int kb = type_size(key_type);
+    if (rows < kSmallRows || bound_picks_hash(rows, group_bound, nops, kb)) {
         // hash, sized by the caller's bound (or the row count)
         *algo = EG_ALGO_HASH;
         if (card_est) *card_est = rows < kSmallRows ? rows : group_bound;
         if (singletons) *singletons = 0.f;
         return true;
     }
-    FQuery q{keys, rows, group_bound, type_size(key_type), nops, value_bytes, 0};
+    const FQuery q = select_query(keys, rows, group_bound, kb, nops, value_bytes);
     {
         KernelTimer timer("mlp_select", s);
         hipLaunchKernelGGL(select_kernel, dim3(1), dim3(kFB), 0, s, q, (const float*)m.params.get<float>(),
@@ -647,7 +662,7 @@ bool mlp_select(const void* keys, int32_t key_type, int64_t rows, int64_t group_
     std::memcpy(h, m.host_out, sizeof h);
     for (float v : h)
         if (!std::isfinite(v)) return false;  // fall back to the rule
-    *algo = algo_of(h, rows);
+    *algo = algo_of(h, rows, nops, kb);
     if (card_est) {
         const double lg = std::min(62.0, std::max(0.0, (double)h[3] * 32.0));
         *card_est = (int64_t)std::min<double>((double)rows, std::exp2(lg));
@@ -833,7 +848,7 @@ int eg_mlp_select_batch(const eg_mlp_query* queries, int64_t num, int32_t* algos
             if (!(u.key_type == EG_INT32 || u.key_type == EG_INT64 || u.key_type == EG_UINT32 || u.key_type == EG_UINT64))
                 eg::raise(EG_ERR_UNSUPPORTED, "features need 4- or 8-byte integer keys");
             if (u.rows < 0 || (u.rows > 0 && !u.keys)) eg::raise(EG_ERR_INVALID, "bad key column");
-            h[(size_t)i] = eg::FQuery{u.keys, u.rows, u.group_bound, eg::type_size(u.key_type), u.nops, u.value_bytes, 0};
+            h[(size_t)i] = eg::select_query(u.keys, u.rows, u.group_bound, eg::type_size(u.key_type), u.nops, u.value_bytes);
         }
         eg::DevBuf dq(h.size() * sizeof(eg::FQuery), s), feat((size_t)num * eg::kIn * 4, s), out((size_t)num * eg::kOut * 4, s);
         EG_HIP(hipMemcpyAsync(dq.get(), h.data(), h.size() * sizeof(eg::FQuery), hipMemcpyHostToDevice, s));
@@ -846,8 +861,10 @@ int eg_mlp_select_batch(const eg_mlp_query* queries, int64_t num, int32_t* algos
         EG_HIP(hipStreamSynchronize(s));
         for (int64_t i = 0; i < num; ++i) {
             const float* o = y.data() + (size_t)i * eg::kOut;
-            const bool by_bound = eg::bound_picks_hash(queries[i].rows, queries[i].group_bound);
-            algos[i] = by_bound ? EG_ALGO_HASH : eg::algo_of(o, queries[i].rows);
+            const eg_mlp_query& u = queries[i];
+            const int kb = eg::type_size(u.key_type);
+            const bool by_bound = eg::bound_picks_hash(u.rows, u.group_bound, u.nops, kb);
+            algos[i] = by_bound ? EG_ALGO_HASH : eg::algo_of(o, u.rows, u.nops, kb);
             if (card_est) {
                 const double lg = std::min(62.0, std::max(0.0, (double)o[3] * 32.0));
                 card_est[i] = queries[i].rows < eg::kSmallRows  // as mlp_select: hash sized by the row count

@@ -150,15 +150,15 @@ def soft_targets(times: np.ndarray, tau: float) -> np.ndarray:
 
 def picks(y: np.ndarray, features: np.ndarray) -> np.ndarray:
     """Strategy index (hash, sort, partition) the library picks from model
-    outputs y: the best class score, except that inputs whose estimated group
-    count, or group bound, is at most 2048 (>= 2^24 rows) or 1280 (>= 2^17
-    rows) go to hash (mlp.hip algo_of, bound_picks_hash)."""
+    outputs y: the best class score, except that inputs of >= 2^17 rows whose
+    estimated group count, or group bound, is at most 2048 go to hash (mlp.hip
+    algo_of, bound_picks_hash; the limit is lower with ten states and more, the
+    traces have two and five)."""
     pick = np.argmax(y[:, :3], axis=1)
     rows = np.exp2(features[:, 0].astype(np.float64) * 32) - 1
     card = np.exp2(np.clip(y[:, 3].astype(np.float64) * 32, 0, 62))
     bound = np.exp2(features[:, 11].astype(np.float64) * 32) - 1
-    limit = np.where(rows >= 2.0 ** 24, 2048.0, 1280.0)
-    return np.where((rows >= 2.0 ** 17) & ((card <= limit) | (bound <= limit + 0.5)), 0, pick)
+    return np.where((rows >= 2.0 ** 17 - 0.5) & ((card <= 2048) | (bound <= 2048.5)), 0, pick)
 
 
 def choice_ms(params: np.ndarray, tr: dict) -> float:

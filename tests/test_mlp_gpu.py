@@ -151,3 +151,55 @@ def test_sizing_of_dispatched_tables(log_rows, bound, algo, card, singles, exp):
     model's estimate, the caller's bound and the full-column estimate."""
     got = G.dispatch_sizing(G.type_id.INT32, 1 << log_rows, bound, 5, 12, G.groupby_algo[algo], card, singles)
     assert got == exp
+
+
+@pytest.mark.parametrize("log_rows,nops,ktype,card,bound,exp", [
+    # card: what the model estimates; it scores PARTITION best
+    (20, 2, np.int32, 2000, 0, "HASH"), (20, 2, np.int32, 2100, 0, "PARTITION"),
+    (24, 2, np.int32, 2000, 0, "HASH"), (24, 2, np.int32, 2100, 0, "PARTITION"),
+    (20, 10, np.int32, 1900, 0, "HASH"), (24, 10, np.int32, 1980, 0, "PARTITION"),     # 1936 slots
+    (20, 16, np.int64, 1150, 0, "HASH"), (20, 16, np.int64, 1260, 0, "PARTITION"),     # ~1200 slots
+    # a caller's bound
+    (20, 2, np.int32, 2100, 2048, "HASH"), (20, 2, np.int32, 2100, 2049, "PARTITION"),
+    (20, 16, np.int32, 2100, 1280, "HASH"), (20, 16, np.int32, 2100, 1281, "PARTITION"),
+    (24, 16, np.int32, 2100, 2048, "HASH"), (24, 16, np.int32, 2100, 2049, "PARTITION"),
+    ((1 << 17) - 1, 2, np.int32, 5000, 0, "HASH"), (17, 2, np.int32, 5000, 0, "PARTITION"),
+])
+def test_hash_by_group_count_depends_on_the_states(log_rows, nops, ktype, card, bound, exp):
+    """A model that always scores partition best and estimates `card`: few
+    enough groups for the LDS table of that many states go to hash."""
+    n = log_rows if log_rows > 64 else 1 << log_rows
+    k = G.make_column(G.to_type_id(ktype), n)
+    P = np.zeros(G.MLP_PARAMS, np.float32)
+    P[5504 + 2] = 5.0
+    P[5507] = np.log2(card) / 32
+    loaded = G.mlp_loaded()
+    G.mlp_load(P)
+    try:
+        algo, _ = G.mlp_select(k, bound, nops=nops, value_bytes=8)
+        assert algo == G.groupby_algo[exp]
+        assert list(G.mlp_select_batch([k], [bound], nops=nops, value_bytes=8)[0]) == [algo]
+    finally:
+        G.mlp_load(None)
+        if loaded:
+            G.load_dispatch_model()
+        k.free()
+
+
+@pytest.mark.parametrize("nops,value_bytes", [(5, 12), (8, 24), (10, 32), (16, 8), (16, 32)])
+@pytest.mark.parametrize("d", [600, 4000, 100_000])
+def test_group_estimates_of_wide_requests(d, nops, value_bytes):
+    """The shipped model's estimate is about the group count (its sizing leaves
+    2.5x headroom) also for requests wider than the ones it was trained on."""
+    k = G.gen_keys_uniform(1 << 20, d, seed=7)
+    loaded = G.mlp_loaded()
+    assert G.load_dispatch_model()
+    try:
+        algo, card = G.mlp_select(k, 0, nops=nops, value_bytes=value_bytes)
+        assert d / 2.5 <= card <= 2.5 * d
+        a, c = G.mlp_select_batch([k], None, nops=nops, value_bytes=value_bytes)
+        assert a[0] == algo and abs(int(c[0]) - card) <= 1 + card // 1000
+    finally:
+        if not loaded:
+            G.mlp_load(None)
+        k.free()

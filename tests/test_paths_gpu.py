@@ -148,9 +148,9 @@ def test_hash_tables_of_many_workgroups_merged(dtype, d, n):
 
 
 @pytest.mark.parametrize("n,bound,d,stored", [
-    (65_536, 400, 400, False), (65_536, 401, 401, True),        # 16 tiles: 16 * bound against 6400 + 16
-    (1 << 20, 25, 25, False), (1 << 20, 26, 20, True),          # 256 tiles: one a compute unit
-    ((1 << 20) + 1, 26, 3, False), ((1 << 20) + 1, 27, 1, True),
+    (65_536, 313, 313, False), (65_536, 314, 314, True),        # 16 tiles: 16 * bound against 5000 + 16
+    (1 << 20, 20, 20, False), (1 << 20, 21, 18, True),          # 256 tiles: one a compute unit
+    ((1 << 20) + 1, 20, 3, False), ((1 << 20) + 1, 21, 1, True),
     (200_003, 16_272, 16_000, True), (200_003, 16_273, 16_000, False),  # twice the LDS slots of two states
 ])
 def test_hash_tables_stored_or_flushed(n, bound, d, stored):
