@@ -11,7 +11,7 @@
 //     (groupby_sort.cu:394-413) is this operation.
 //
 // The dictionary goes into an open-addressing table of 2^c slots (m dictionary
-// entries, at most 3/4 full): slot value = dictionary position + 1 (0 = empty,
+// entries, at most 5/8 full): slot value = dictionary position + 1 (0 = empty,
 // so a zero-fill clears it), claimed by compare-and-swap; a duplicate key
 // keeps its smallest position (atomicMin), so results are deterministic.  A
 // second pass stores each slot's key beside it.  The lookup streams the column
@@ -34,10 +34,12 @@ namespace {
 constexpr int kDictBlock = 1024;
 constexpr int kLdsSlotsMax = 8192;  // 32 KB of positions + up to 64 KB of keys
 constexpr int64_t kMaxDict = (int64_t)1 << 30;
+// HBM tables of 16-byte slots from this size on (16 MB) are read two slots a step.
+constexpr int kPairSlotsLog2 = 20;
 
 // First slot of the key's bucket: buckets are aligned groups of 2^align slots
 // that one step of a lookup reads (the LDS table 4, the HBM table 2 of 8
-// bytes or 1 of 16), and probing runs linearly from there.  Keys of up to 4
+// bytes, 1 of 16 or 2 of 16), and probing runs linearly from there.  Keys of up to 4
 // bytes take the 32-bit mixer (a third of the multiplies of the 64-bit one).
 template <bool WIDE>
 __device__ __forceinline__ uint32_t dict_home(uint64_t raw, int cap_log2, int align)
@@ -238,15 +240,21 @@ __global__ __launch_bounds__(kDictBlock) void dict_find_lds_kernel(const void* _
 // decided read on; the key and id streams are non-temporal so the table keeps
 // the L2.  Reading a 64-byte bucket of four 16-byte slots for every row took
 // 1.39 ms for 100M int32 rows and 300k keys.
-template <int KB, int OB>
+// W: 16-byte pieces a step reads.  Two for large tables of 16-byte slots, where
+// a step's latency counts for more than its requests (100M int64 rows, half of
+// them absent, 2^23 slots 0.4 full: 3.19 ms with one, 2.52 with two; 2^19 slots
+// 1.35 and 1.44).
+template <int KB, int OB, int W>
 __global__ __launch_bounds__(kDictBlock) void dict_find_hbm_kernel(const void* __restrict__ keys, int64_t n,
                                                                    const uint4* __restrict__ table, int cap_log2,
                                                                    uint64_t miss, void* __restrict__ out)
 {
     constexpr bool kWide = KB > 4;
-    constexpr int kAlign = kWide ? 0 : 1;  // log2 slots per 16 bytes
-    constexpr int U = 4;                   // rows in flight per lane
-    const uint32_t mask = (1u << (cap_log2 - kAlign)) - 1u;  // in 16-byte steps
+    static_assert(W == 1 || (W == 2 && kWide), "pieces of a step");
+    constexpr int kAlign = kWide ? 0 : 1;   // log2 slots per 16 bytes
+    constexpr int kHome = kAlign + W - 1;   // log2 slots per step
+    constexpr int U = 4;                    // rows in flight per lane
+    const uint32_t mask = (1u << (cap_log2 - kAlign)) - 1u;  // in 16-byte pieces
     using KT = typename std::conditional<KB == 1, uint8_t, typename std::conditional<KB == 2, uint16_t,
                typename std::conditional<KB == 4, uint32_t, unsigned long long>::type>::type>::type;
     using OT = typename std::conditional<OB == 1, uint8_t, typename std::conditional<OB == 2, uint16_t,
@@ -260,31 +268,38 @@ __global__ __launch_bounds__(kDictBlock) void dict_find_hbm_kernel(const void* _
             const int64_t r = i + u * stride;
             k[u] = r < n ? (uint64_t)__builtin_nontemporal_load((const KT*)keys + r) : 0ull;
             if (r < n) open |= 1u << u;
-            h[u] = dict_home<kWide>(k[u], cap_log2, kAlign) >> kAlign;
+            h[u] = dict_home<kWide>(k[u], cap_log2, kHome) >> kAlign;
             res[u] = miss;
         }
         // an empty slot ends every probe sequence (the table is never full)
         while (open) {
-            uint4 b[U];
+            uint4 b[U][W];
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                if ((open >> u) & 1u) b[u] = table[h[u]];
+                if ((open >> u) & 1u) {
+#pragma unroll
+                    for (int j = 0; j < W; ++j) b[u][j] = table[h[u] + j];  // a step's pieces are aligned together
+                }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                if (!((open >> u) & 1u)) continue;
-                uint32_t pos = 0u;
-                bool end;
-                if constexpr (kWide) {
-                    if ((((uint64_t)b[u].y << 32) | b[u].x) == k[u]) pos = b[u].z;
-                    end = b[u].z == 0u;
-                } else {
-                    if (b[u].x == (uint32_t)k[u]) pos = b[u].y;  // 0 in an empty slot
-                    else if (b[u].z == (uint32_t)k[u]) pos = b[u].w;
-                    end = b[u].y == 0u || b[u].w == 0u;
+#pragma unroll
+                for (int j = 0; j < W; ++j) {
+                    if (!((open >> u) & 1u)) break;
+                    const uint4 t = b[u][j];
+                    uint32_t pos = 0u;
+                    bool end;
+                    if constexpr (kWide) {
+                        if ((((uint64_t)t.y << 32) | t.x) == k[u]) pos = t.z;
+                        end = t.z == 0u;
+                    } else {
+                        if (t.x == (uint32_t)k[u]) pos = t.y;  // 0 in an empty slot
+                        else if (t.z == (uint32_t)k[u]) pos = t.w;
+                        end = t.y == 0u || t.w == 0u;
+                    }
+                    if (pos) res[u] = pos - 1u;
+                    if (pos || end) open &= ~(1u << u);
                 }
-                if (pos) res[u] = pos - 1u;
-                if (pos || end) open &= ~(1u << u);
-                h[u] = (h[u] + 1u) & mask;
+                h[u] = (h[u] + (uint32_t)W) & mask;
             }
         }
 #pragma unroll
@@ -372,7 +387,11 @@ template <int KB, int OB>
 void launch_find(bool in_lds, const void* keys, int64_t n, const uint32_t* slots, const void* aux, int cap_log2,
                  uint64_t miss, void* out, hipStream_t s)
 {
-    const void* kern = in_lds ? (const void*)dict_find_lds_kernel<KB, OB> : (const void*)dict_find_hbm_kernel<KB, OB>;
+    const bool pairs = KB > 4 && cap_log2 >= kPairSlotsLog2;
+    auto hbm = dict_find_hbm_kernel<KB, OB, 1>;
+    if constexpr (KB > 4)
+        if (pairs) hbm = dict_find_hbm_kernel<KB, OB, 2>;
+    const void* kern = in_lds ? (const void*)dict_find_lds_kernel<KB, OB> : (const void*)hbm;
     size_t lds = 0;
     if (in_lds) {
         lds = ((size_t)4 + sizeof(SlotKey<KB>)) << cap_log2;
@@ -387,7 +406,7 @@ void launch_find(bool in_lds, const void* keys, int64_t n, const uint32_t* slots
         hipLaunchKernelGGL((dict_find_lds_kernel<KB, OB>), dim3((unsigned)grid), dim3(kDictBlock), lds, s, keys, n, slots,
                            (const uint64_t*)aux, cap_log2, miss, out);
     else
-        hipLaunchKernelGGL((dict_find_hbm_kernel<KB, OB>), dim3((unsigned)grid), dim3(kDictBlock), 0, s, keys, n,
+        hipLaunchKernelGGL(hbm, dim3((unsigned)grid), dim3(kDictBlock), 0, s, keys, n,
                            (const uint4*)aux, cap_log2, miss, out);
     EG_LAUNCH_CHECK();
 }
@@ -478,11 +497,16 @@ DevBuf dict_encode(const void* keys, int64_t n, const void* dict, int64_t m, int
     int cap_log2 = 6;
     while (((int64_t)1 << cap_log2) < 2 * m) ++cap_log2;
     const bool in_lds = ((int64_t)1 << cap_log2) <= kLdsSlotsMax;
-    // an HBM table up to 3/4 full: half the size keeps more of it in the L2
-    // than the longer probes cost (300k int32 keys, 100M rows: 4 MB 0.92 ms, 8 MB 0.96)
-    if (!in_lds && 4 * m <= (int64_t)3 << (cap_log2 - 1)) --cap_log2;
+    // at most half full, except that 8-byte slots may fill 4 MB to 3/5 and 8 MB to
+    // 5/8: the next size would leave the 4 MB L2 or be twice as far out of it,
+    // which costs more than the longer probes (100M rows, every key present,
+    // 0.58 full 4 MB 0.94 ms, 8 MB 0.96; 8 MB 1.16, 16 MB 1.45).  Elsewhere they
+    // cost more: 0.3 of 128 KB 644 us, 0.6 of 64 KB 818; 16-byte slots, 0.28 of 2^18
+    // 844 us, 0.56 of 2^17 1117, 0.37 of 2^22 1.6 ms, 0.74 of 2^21 2.6.
+    const int64_t smaller = (int64_t)1 << (cap_log2 - 1);
+    if (!wide && ((cap_log2 == 20 && 5 * m <= 3 * smaller) || (cap_log2 == 21 && 8 * m <= 5 * smaller))) --cap_log2;
     const int64_t cap = (int64_t)1 << cap_log2;
-    const int align = in_lds ? 2 : wide ? 0 : 1;
+    const int align = in_lds ? 2 : wide ? (cap_log2 >= kPairSlotsLog2 ? 1 : 0) : 1;
     DevBuf slots((size_t)cap * 4, s);
     fill_zero(slots.get(), (size_t)cap * 4, s);
     DevBuf aux((size_t)cap * (in_lds || !wide ? 8 : 16), s);

@@ -92,6 +92,23 @@ def test_dictionary_table_sizes_around_the_lds_limit_and_load(dtype, m):
     np.testing.assert_array_equal(got, O.dict_encode(keys, pool))
 
 
+@pytest.mark.parametrize("dtype,m", [
+    (np.int32, 314_572), (np.int32, 314_573), (np.int32, 655_360), (np.int32, 655_361),  # 3/5 of 2^19, 5/8 of 2^20 slots
+    (np.int64, 262_144), (np.int64, 262_145), (np.int64, 524_289)])  # 2^19, 2^20, 2^21 slots: one, two a step
+def test_dictionary_table_sizes_around_the_l2(dtype, m):
+    """Large dictionaries on both sides of the lines between table sizes and
+    between one and two slots a step; half of the keys are absent."""
+    rng = np.random.default_rng(m)
+    info = np.iinfo(dtype)
+    pool = rng.integers(info.min, info.max, m, dtype=dtype, endpoint=True)
+    pool[0], pool[1] = info.min, info.max
+    n = 600_011
+    keys = np.where(rng.random(n) < 0.5, rng.choice(pool, n), rng.integers(info.min, info.max, n, dtype=dtype, endpoint=True)).astype(dtype)
+    kc, dc = G.make_column_from_host(keys), G.make_column_from_host(pool)
+    got = G.dictionary_encode_with_dict(kc, dc).to_numpy()
+    np.testing.assert_array_equal(got, O.dict_encode(keys, pool))
+
+
 @pytest.mark.parametrize("bits", [(16, 16), (17, 16), (1, 31), (32,), (33,), (8, 8, 8, 8)])
 @pytest.mark.parametrize("algo", ["AUTO_ALGO", "HASH", "SORT", "PARTITION"])
 def test_fused_keys_around_32_bits(bits, algo):
