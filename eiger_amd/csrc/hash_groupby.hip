@@ -96,12 +96,14 @@ void launch_compact(const GTable& gt, const OutSpec& os, unsigned long long* cou
 // 2^20, 16 52/49, 1000 306/60; 2^26, 64 248/244, 128 274/246; 2^28 (five
 // states), 16 766/832, 200 789/796, 400 891/808.  Above two value columns a
 // block has half the threads: 2^26 rows, 12 states, 100 groups 1025/1100.
+// Below 16 blocks a flush meets little: 16,000 rows of unknown groups, ten of
+// them 42/47, 1000 of them 57/63.
 bool store_pays(int64_t rows, int64_t groups, int nvcols)
 {
     const int64_t tile = nvcols <= 2 ? 4096 : 2048;
     const int64_t tiles = (rows + tile - 1) / tile;
     const int64_t blocks = std::min<int64_t>(tiles, device_info().num_cus);
-    return blocks * groups >= 5000 + tiles;
+    return blocks >= 16 && blocks * groups >= 5000 + tiles;
 }
 
 // The aggregation of n rows into gt.  `scratch` (optional): where the blocks'

@@ -165,6 +165,7 @@ def test_hash_tables_of_many_workgroups_merged(dtype, d, n):
 
 
 @pytest.mark.parametrize("n,bound,d,stored", [
+    (61_440, 8000, 500, False), (61_441, 8000, 500, True),      # 15 and 16 blocks
     (65_536, 313, 313, False), (65_536, 314, 314, True),        # 16 tiles: 16 * bound against 5000 + 16
     (1 << 20, 20, 20, False), (1 << 20, 21, 18, True),          # 256 tiles: one a compute unit
     ((1 << 20) + 1, 20, 3, False), ((1 << 20) + 1, 21, 1, True),
