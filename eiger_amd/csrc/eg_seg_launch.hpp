@@ -12,6 +12,8 @@ namespace eg {
 constexpr int kSegB = 256;
 // 2048-row tiles: the turned column and five states leave five workgroups a CU.
 constexpr int kSegItems = 8;
+// Tiles that add to one address when a group covers them all.
+constexpr uint32_t kSegSpan = 128;
 
 // Requests of at most this many states take kernels unrolled for that many,
 // half the code and 67 instead of 88 registers (40M rows of int64 keys and

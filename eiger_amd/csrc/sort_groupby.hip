@@ -67,15 +67,53 @@ __global__ __launch_bounds__(kSegB) void seg_heads_kernel(const void* __restrict
     if (threadIdx.x == 0) heads[blockIdx.x] = ws[0] + ws[1] + ws[2] + ws[3];
 }
 
-__global__ void seg_tail_kernel(uint32_t ntiles, const uint32_t* head_off, const unsigned long long* bstate,
-                                const unsigned long long* bkey, const uint32_t* btrail, int nops, int kb,
+// Writes the groups that continue past the tile of their head (one lane per
+// tile).  A group that covers the first tile of later spans has a partial
+// state at each of those: the wave collects them.  Such a group covers all
+// tiles from its head's to the next span's first, so a wave's 64 tiles hold
+// the head of at most one.
+__global__ void seg_tail_kernel(uint32_t ntiles, const uint32_t* head_off, unsigned long long* bstate,
+                                const unsigned long long* bkey, const uint32_t* btrail, AggSpec spec, int kb,
                                 int is_signed, OutSpec os)
 {
+    const int nops = spec.nops;
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ntiles || btrail[t] == 0u) return;
-    const uint32_t gidx = head_off[t + 1] - 1u;
-    dev::emit_group(os, (int64_t)gidx, dev::enc64(dev::widen_key(bkey[t], kb, is_signed)), bstate + (size_t)t * nops,
-                    (int64_t)1);
+    const int lane = threadIdx.x & 63;
+    const bool trail = t < ntiles && btrail[t] != 0u;
+    const uint32_t groups = trail ? head_off[t + 1] : 0u;  // this one is the last of them
+    const uint32_t next = (t & ~(kSegSpan - 1u)) + kSegSpan;
+    const bool spans = trail && next < ntiles && head_off[next + 1] == groups;
+    if (const uint64_t m = __ballot(spans)) {
+        const int src = __ffsll((unsigned long long)m) - 1;
+        const uint32_t g = __shfl(groups, src), first = __shfl(next, src);
+        for (int a = 0; a < nops; ++a) {
+            const int32_t cls = dev::class_of(spec, a);
+            uint64_t v = 0ull;
+            int have = 0;
+            for (uint64_t s = first + (uint64_t)lane * kSegSpan; s < ntiles && head_off[s + 1] == g; s += 64 * kSegSpan) {
+                const uint64_t x = bstate[(size_t)s * nops + a];
+                v = have ? dev::combine(cls, v, x) : x;
+                have = 1;
+            }
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) {
+                const uint64_t x = __shfl_down((unsigned long long)v, off);
+                const int other = __shfl_down(have, off);
+                if (lane + off < 64 && other) {
+                    v = have ? dev::combine(cls, v, x) : x;
+                    have = 1;
+                }
+            }
+            v = __shfl((unsigned long long)v, 0);
+            if (lane == src) {
+                unsigned long long* dst = bstate + (size_t)t * nops + a;
+                *dst = dev::combine(cls, *dst, v);
+            }
+        }
+    }
+    if (trail)
+        dev::emit_group(os, (int64_t)groups - 1, dev::enc64(dev::widen_key(bkey[t], kb, is_signed)),
+                        bstate + (size_t)t * nops, (int64_t)1);
 }
 
 }  // namespace
@@ -118,9 +156,9 @@ Result reduce_sorted(const Plan& plan, const void* sorted_keys, const AggSpec& s
     if (kb == 4) (few ? launch_seg<4, kSegFewOps> : launch_seg<4, kMaxOps>)(sa, sg, spec, os, s);
     else (few ? launch_seg<8, kSegFewOps> : launch_seg<8, kMaxOps>)(sa, sg, spec, os, s);
     hipLaunchKernelGGL(seg_tail_kernel, dim3((ntiles + 255) / 256), dim3(256), 0, s, ntiles,
-                       (const uint32_t*)head_off.get<uint32_t>(), (const unsigned long long*)bstate.get<unsigned long long>(),
+                       (const uint32_t*)head_off.get<uint32_t>(), bstate.get<unsigned long long>(),
                        (const unsigned long long*)bkey.get<unsigned long long>(), (const uint32_t*)btrail.get<uint32_t>(),
-                       spec.nops, kb, sg, os);
+                       spec, kb, sg, os);
     EG_LAUNCH_CHECK();
     EG_HIP(hipStreamSynchronize(s));
     return res;

@@ -280,3 +280,20 @@ def _check_partitioned(n, d, bound, states, passes):
         G.kernel_timing(False)
         G.kernel_timing_reset()
     assert_same(got, exp)
+
+
+@pytest.mark.parametrize("before,rows,after", [
+    (b, r, a) for b in (0, 1, 2048, 126 * 2048 + 5, 128 * 2048 - 1, 128 * 2048)
+    for r, a in ((128 * 2048, 0), (128 * 2048 + 1, 1), (258 * 2048 + 3, 130 * 2048))] + [(77, 66 * 128 * 2048, 3)])
+def test_sort_groups_longer_than_a_span_of_tiles(before, rows, after):
+    """One group of more rows than 128 tiles of 2048, its head in, at and
+    around the first tile of a span, with groups before and after it."""
+    rng = np.random.default_rng(before + rows + after)
+    keys = np.concatenate([np.sort(rng.integers(0, 5, before)), np.full(rows, 7), 9 + np.sort(rng.integers(0, 3, after))])
+    keys = keys.astype(np.int32)
+    a = rng.integers(-1000, 1000, len(keys)).astype(np.int64)
+    one = (keys * 3).astype(np.int32)  # one value per key
+    reqs = [(0, A.SUM), (0, A.MIN), (0, A.MAX), (-1, A.COUNT_ALL), (1, A.ANY)]
+    exp = sorted_by_key(O.groupby(keys, [a, one], reqs))
+    for fn in (G.sort_groupby, G.sort_groupby_gfur):
+        assert_same(run(fn, keys, [a, one], reqs), exp)
