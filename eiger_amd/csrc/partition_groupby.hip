@@ -153,64 +153,43 @@ __global__ __launch_bounds__(256) void units_fill_kernel(const int64_t* __restri
 }
 
 // Boundaries and units of up to kUnitsSmall partitions in one launch of one
-// workgroup (five launches otherwise): thread t finds the first rows of its
-// consecutive partitions by binary search, then one scan places the units.
-// Above, one CU's searches take longer than the launches (4096 partitions of
-// 2^28 rows: 168 us against ~35).
-constexpr int kUnitsPer = 1;
-constexpr int64_t kUnitsSmall = 512;
+// workgroup (five launches otherwise): thread t finds partition t's first row
+// by binary search, then one scan places the units.  Above, one CU's searches
+// take longer than the launches (4096 partitions of 2^28 rows: 168 us against
+// ~35).
+constexpr int kUnitsSmall = 512;
 
 template <int KB>
-__global__ __launch_bounds__(1024) void units_small_kernel(const void* __restrict__ keys, int64_t n, uint32_t mask,
-                                                           int64_t P, int64_t whole, int64_t slice,
-                                                           agg::Unit* __restrict__ units, unsigned long long* meta)
+__global__ __launch_bounds__(kUnitsSmall) void units_small_kernel(const void* __restrict__ keys, int64_t n, uint32_t mask,
+                                                                  int P, int64_t whole, int64_t slice,
+                                                                  agg::Unit* __restrict__ units, unsigned long long* meta)
 {
-    __shared__ uint32_t wsum[16];
+    __shared__ uint32_t wsum[kUnitsSmall / 64];
     __shared__ int64_t first[kUnitsSmall + 1];
     __shared__ uint32_t s_sliced;
     const int t = threadIdx.x;
-    const int per = (int)((P + 1023) / 1024);
     if (t == 0) s_sliced = 0u;
-    int64_t lo[kUnitsPer], hi[kUnitsPer];
-#pragma unroll
-    for (int i = 0; i < kUnitsPer; ++i) lo[i] = 0, hi[i] = i < per && (int64_t)t * per + i < P ? n : 0;
-    bool more = true;
-    while (more) {  // rows < lo have id < p, rows >= hi have id >= p; the searches side by side
-        more = false;
-#pragma unroll
-        for (int i = 0; i < kUnitsPer; ++i) {
-            if (lo[i] >= hi[i]) continue;
-            const int64_t mid = lo[i] + ((hi[i] - lo[i]) >> 1);
-            if ((int64_t)pid_of<KB>(dev::load_raw(keys, KB, mid), mask) < (int64_t)t * per + i) lo[i] = mid + 1;
-            else hi[i] = mid;
-            more = more || lo[i] < hi[i];
-        }
+    int64_t lo = 0, hi = t < P ? n : 0;
+    while (lo < hi) {  // rows < lo have id < t, rows >= hi have id >= t
+        const int64_t mid = lo + ((hi - lo) >> 1);
+        if ((int)pid_of<KB>(dev::load_raw(keys, KB, mid), mask) < t) lo = mid + 1;
+        else hi = mid;
     }
-#pragma unroll
-    for (int i = 0; i < kUnitsPer; ++i)
-        if (i < per && (int64_t)t * per + i < P) first[t * per + i] = lo[i];
+    if (t < P) first[t] = lo;
     if (t == 0) first[P] = n;
     __syncthreads();
-    uint32_t cnt[kUnitsPer], sum = 0, sliced = 0;
-#pragma unroll
-    for (int i = 0; i < kUnitsPer; ++i) {
-        cnt[i] = 0;
-        if (i < per && (int64_t)t * per + i < P) {
-            const int64_t rows = first[t * per + i + 1] - first[t * per + i];
-            cnt[i] = rows <= 0 ? 0u : rows <= whole ? 1u : (uint32_t)((rows + slice - 1) / slice);
-            sliced += rows > whole ? 1u : 0u;
-        }
-        sum += cnt[i];
+    uint32_t cnt = 0;
+    if (t < P) {
+        const int64_t rows = first[t + 1] - lo;
+        cnt = rows <= 0 ? 0u : rows <= whole ? 1u : (uint32_t)((rows + slice - 1) / slice);
+        if (rows > whole) atomicAdd(&s_sliced, 1u);
     }
-    if (sliced) atomicAdd(&s_sliced, sliced);
-    uint32_t at = dev::block_excl_scan<1024>(sum, wsum);
-    if (t == 1023) meta[1] = (unsigned long long)at + sum;
-#pragma unroll
-    for (int i = 0; i < kUnitsPer; ++i)
-        for (uint32_t j = 0; j < cnt[i]; ++j) {
-            const int64_t x = first[t * per + i] + (int64_t)j * slice, e = first[t * per + i + 1];
-            units[at++] = agg::Unit{x, cnt[i] == 1 ? e : (x + slice < e ? x + slice : e), cnt[i] > 1 ? 1 : 0, 0};
-        }
+    const uint32_t at = dev::block_excl_scan<kUnitsSmall>(cnt, wsum);
+    if (t == kUnitsSmall - 1) meta[1] = (unsigned long long)at + cnt;
+    for (uint32_t j = 0; j < cnt; ++j) {
+        const int64_t x = lo + (int64_t)j * slice, e = first[t + 1];
+        units[at + j] = agg::Unit{x, cnt == 1 ? e : (x + slice < e ? x + slice : e), cnt > 1 ? 1 : 0, 0};
+    }
     __syncthreads();
     if (t == 0) meta[0] = s_sliced;
 }
@@ -447,8 +426,8 @@ Result run_partition(const Plan& plan, int64_t group_bound, int64_t expected, bo
         if (P <= kUnitsSmall) {
             KernelTimer timer("partition_bounds", s);
             auto kern = kb == 4 ? units_small_kernel<4> : units_small_kernel<8>;
-            hipLaunchKernelGGL(kern, dim3(1), dim3(1024), 0, s, pkeys, n, pmask, P, whole, slice, dunits.get<Unit>(),
-                               umeta);
+            hipLaunchKernelGGL(kern, dim3(1), dim3(kUnitsSmall), 0, s, pkeys, n, pmask, (int)P, whole, slice,
+                               dunits.get<Unit>(), umeta);
             EG_LAUNCH_CHECK();
         } else {
             offs = DevBuf((size_t)(P + 1) * 8, s);

@@ -576,21 +576,21 @@ void radix_pass(const RadixKeys& k, void* keys_out, const std::vector<Payload>& 
                                ntiles, nd, offs.get<uint32_t>());
             EG_LAUNCH_CHECK();
         } else {
-        const int per = std::max(16, (ntiles + 4095) / 4096);  // tiles per chunk: at most 4096 chunks
-        const int nchunks = (ntiles + per - 1) / per;
-        DevBuf cs((size_t)nchunks * nd * 4 * 2 + (size_t)nd * 4, s);
-        uint32_t* csum = cs.get<uint32_t>();
-        uint32_t* coff = csum + (size_t)nchunks * nd;
-        uint32_t* total = coff + (size_t)nchunks * nd;
-        hipLaunchKernelGGL(tile_chunk_sums_kernel, dim3(nchunks), dim3(kOB), 0, s, (const uint32_t*)hist.get<uint32_t>(),
-                           ntiles, nd, per, csum);
-        EG_LAUNCH_CHECK();
-        hipLaunchKernelGGL(tile_chunk_scan_kernel, dim3(nd), dim3(1024), 0, s, (const uint32_t*)csum, nchunks, nd, coff,
-                           total);
-        EG_LAUNCH_CHECK();
-        hipLaunchKernelGGL(tile_offsets_kernel, dim3(nchunks), dim3(kOB), 0, s, (const uint32_t*)hist.get<uint32_t>(),
-                           ntiles, nd, per, (const uint32_t*)coff, (const uint32_t*)total, offs.get<uint32_t>());
-        EG_LAUNCH_CHECK();
+            const int per = std::max(16, (ntiles + 4095) / 4096);  // tiles per chunk: at most 4096 chunks
+            const int nchunks = (ntiles + per - 1) / per;
+            DevBuf cs((size_t)nchunks * nd * 4 * 2 + (size_t)nd * 4, s);
+            uint32_t* csum = cs.get<uint32_t>();
+            uint32_t* coff = csum + (size_t)nchunks * nd;
+            uint32_t* total = coff + (size_t)nchunks * nd;
+            hipLaunchKernelGGL(tile_chunk_sums_kernel, dim3(nchunks), dim3(kOB), 0, s, (const uint32_t*)hist.get<uint32_t>(),
+                               ntiles, nd, per, csum);
+            EG_LAUNCH_CHECK();
+            hipLaunchKernelGGL(tile_chunk_scan_kernel, dim3(nd), dim3(1024), 0, s, (const uint32_t*)csum, nchunks, nd, coff,
+                               total);
+            EG_LAUNCH_CHECK();
+            hipLaunchKernelGGL(tile_offsets_kernel, dim3(nchunks), dim3(kOB), 0, s, (const uint32_t*)hist.get<uint32_t>(),
+                               ntiles, nd, per, (const uint32_t*)coff, (const uint32_t*)total, offs.get<uint32_t>());
+            EG_LAUNCH_CHECK();
         }
     }
     PayArgs pa{};

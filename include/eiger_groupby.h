@@ -449,11 +449,13 @@ int eg_jit_wait(void);
 int eg_jit_stats(int64_t* out6);
 /* Queues, on the background compiler thread, the hash and partition
  * aggregation kernels specialised for this request list (key type, value
- * column types, requests as eg_groupby lowers them), for `arch` (e.g.
+ * column types, requests as eg_groupby lowers them; UINT64 keys also queue the
+ * 4-byte kernels that fused keys of up to 32 bits take), for `arch` (e.g.
  * "gfx950:sramecc+:xnack-", the device's gcnArchName; NULL = the current
  * device's).  Needs no device when `arch` is given.  Lets a caller warm the
  * specialisation cache before its data arrives; *queued (may be NULL) = the
- * number of new compiles.  A process may exit with compiles queued or
+ * number of new compiles (the hash aggregation's two kernels, storing and
+ * flushing its tables, are one).  A process may exit with compiles queued or
  * running. */
 int eg_jit_prefetch(int32_t key_type, const int32_t* val_types, int64_t num_vals,
                     const eg_agg_request* reqs, int64_t num_reqs, const char* arch,

@@ -217,9 +217,9 @@ def test_tiny_inputs_in_one_workgroup(n, ktype):
 
 @pytest.mark.parametrize("bound", [300, 100_000, 390_000, 1_100_000])
 def test_partition_counts_around_the_one_launch_unit_list(bound):
-    """Bounds that give a few, about 100, 256 (one digit pass, fuller tables)
-    and more than 512 partitions, over keys far fewer than the bound with one
-    key that most rows hold (its partition is sliced)."""
+    """Bounds that give 2, 64, 256 and 1024 partitions (one launch makes the
+    unit list of up to 512), over keys far fewer than the bound with one key
+    that most rows hold (its partition is sliced)."""
     n = 1_200_007
     keys = O.gen_keys_uniform(n, 20_011, seed=bound)
     keys[np.random.default_rng(3).random(n) < 0.6] = 77
