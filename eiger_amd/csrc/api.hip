@@ -317,22 +317,27 @@ struct GroupSizing {
 // smaller estimate replaces it: the model's estimate with 2.5x headroom.  On
 // inputs of 2^24 rows or more whose sample is mostly singletons (more than 1/4
 // of its keys seen once) the model's estimate can be too low by more than the
-// headroom (up to 3.3x over 2^24 to 2^28 rows in 2^11 to 2^26 keys), and the
-// full-column HyperLogLog estimate (standard error 0.8%, 25% headroom) sizes
-// the tables instead: one pass over the keys (0.25 ms per 2^28 rows and a
+// headroom (2^28 rows in 2^22 groups: 0.45M with that bound, 0.94M without),
+// and the full-column HyperLogLog estimate (standard error 0.8%, 25% headroom)
+// sizes the tables instead: one pass over the keys (0.25 ms per 2^28 rows and a
 // synchronisation), cheap against such an input, and tighter tables.
 // - With no caller bound it runs whatever the estimate (67M rows in 16.7M
 //   groups were cut into 32768 partitions for the row count as bound: 2.98 ->
 //   2.75 ms).
-// - With one, and the partition strategy, only where the tighter bound saves
-//   enough: a radix pass; digit bits, where rows times bits reach 2^27 (2^28
-//   rows with 2^18 as bound, in 2^13 groups 4.3 ms without the estimate, 3.5
-//   with it, in 2^16 groups, which saves no bit, 3.86 / 3.75; 2^24 rows in 2^13
-//   groups 0.46 / 0.57), of one pass of less than 8 bits 2^29 (2^28 rows, 2^17 as
-//   bound for 2^15 groups 3.92 / 4.19); or where the partitions of two passes
+// - With one, and the partition strategy, the caller's bound stands unless the
+//   tighter one saves enough: a radix pass; where the partitions of two passes
 //   are so small (16384 rows) that fewer of them make a faster unit kernel
 //   (2^28 rows, Zipf 1.0, 2^26 as bound for 30M groups: 8.0 ms without, 7.4
-//   with).  Else the caller's bound stands.
+//   with it); or digit bits, if the model's bound is below a quarter of the
+//   caller's.  Above, it may only be short of a tight one (2^28 rows, 2^22
+//   groups and bound: 6.03 ms, with a HyperLogLog pass that saves nothing 6.29;
+//   Zipf 1.2, few singletons, the estimate overrun and the aggregation
+//   repeated, 7.46).
+// - For digit bits the pass has to pay for itself: rows times bits reach 2^27
+//   (2^28 rows with 2^18 as bound, in 2^13 groups 4.3 ms without the estimate,
+//   3.5 with it, in 2^16 groups, which saves no bit, 3.86 / 3.75; 2^24 rows in
+//   2^13 groups 0.46 / 0.57), for one pass of less than 8 bits 2^29 (2^28 rows,
+//   2^17 as bound for 2^15 groups 3.92 / 4.19).
 // Below 2^24 rows the pass and its synchronisation would cost more than the
 // tighter sizing saves; the model's estimate stays within 1.34x of the true
 // count on every held-out query of that kind (2,913), far inside the headroom.
@@ -341,15 +346,16 @@ GroupSizing dispatch_sizing(const Plan& plan, int algo, int64_t group_bound, int
     const bool known = group_bound > 0 && group_bound < plan.rows;
     GroupSizing z{known ? group_bound : plan.rows, 0, card, false};
     z.bound = std::min<int64_t>(z.caller, card + card + card / 2 + 1024);
-    z.full_estimate = plan.rows >= ((int64_t)1 << 24) && singletons > 0.25f && (z.bound < z.caller || !known);
-    if (!z.full_estimate || !known || algo != EG_ALGO_PARTITION) return z;
+    if (plan.rows < ((int64_t)1 << 24)) return z;
+    z.full_estimate = singletons > 0.25f && (z.bound < z.caller || !known);
+    if (!known || algo != EG_ALGO_PARTITION || z.bound >= z.caller) return z;
     const PartitionShape loose = partition_shape(plan, z.caller, z.bound), tight = partition_shape(plan, z.bound, card);
     const int64_t worth = (int64_t)1 << (loose.bits < 8 ? 29 : 27);
-    z.full_estimate = loose.passes != tight.passes || (loose.bits - tight.bits) * plan.rows >= worth ||
-                      (loose.passes > 1 && loose.part_rows < 16384);
-    if (!z.full_estimate) {
+    const bool bits = z.bound < z.caller / 4 && (!z.full_estimate || (loose.bits - tight.bits) * plan.rows >= worth);
+    if (loose.passes == tight.passes && !bits && !(loose.passes > 1 && loose.part_rows < 16384)) {
         z.expected = z.bound;
         z.bound = z.caller;
+        z.full_estimate = false;
     }
     return z;
 }

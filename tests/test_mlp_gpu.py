@@ -134,12 +134,16 @@ def test_batched_selection_equals_single_query_selection():
     (20, 1 << 18, "PARTITION", 10_000, 0.9, (26_024, 10_000, False)),
     (20, 20_000, "PARTITION", 10_000, 0.9, (20_000, 10_000, False)),
     (24, 1 << 18, "PARTITION", 10_000, 0.2, (26_024, 10_000, False)),     # few singletons: the estimate stands
-    (28, 1 << 24, "PARTITION", 2_000_000, 0.2, (5_001_024, 2_000_000, False)),
+    (28, 1 << 24, "PARTITION", 1_500_000, 0.2, (3_751_024, 1_500_000, False)),
+    (28, 1 << 24, "PARTITION", 2_000_000, 0.2, (1 << 24, 5_001_024, False)),  # perhaps short of a tight bound
     (24, 1 << 18, "PARTITION", 10_000, 0.9, (1 << 18, 26_024, False)),    # 2^24 rows: three digit bits do not pay
     (28, 1 << 18, "PARTITION", 10_000, 0.9, (26_024, 10_000, True)),      # 2^28 rows: they do
     (28, 1 << 18, "PARTITION", 100_000, 0.9, (1 << 18, 251_024, False)),  # no digit bit saved
     (28, 1 << 17, "PARTITION", 25_000, 0.9, (1 << 17, 63_524, False)),    # seven bits to six
     (28, 1 << 22, "PARTITION", 50_000, 0.9, (126_024, 50_000, True)),     # a pass saved
+    (28, 1 << 22, "PARTITION", 452_975, 1.0, (1 << 22, 1_133_461, False)),  # the same, of singletons
+    (28, 1 << 22, "PARTITION", 415_000, 1.0, (1_038_524, 415_000, True)),   # below a quarter of it
+    (28, 1 << 18, "PARTITION", 61_752, 1.0, (1 << 18, 155_404, False)),
     (28, 1 << 24, "PARTITION", 6_000_000, 0.9, (1 << 24, 15_001_024, False)),
     (28, 1 << 26, "PARTITION", 20_000_000, 0.9, (50_001_024, 20_000_000, True)),  # small partitions
     (28, 1 << 18, "HASH", 10_000, 0.9, (26_024, 10_000, True)),
