@@ -461,6 +461,7 @@ int groupby_entry(Entry entry, const eg_column_view* keys, int64_t num_keys,
         int algo;
         int64_t group_bound = 0;  // from the dispatch model's estimate, else from the hint
         int64_t expected = 0;     // the estimate itself, else the bound
+        const bool callers = h.groups_upper_bound > 0 && h.groups_upper_bound < plan.rows;
         switch (entry) {
         case Entry::HASH: algo = EG_ALGO_HASH; break;
         case Entry::SORT: algo = EG_ALGO_SORT; break;
@@ -507,7 +508,7 @@ int groupby_entry(Entry entry, const eg_column_view* keys, int64_t num_keys,
                 if (group_bound == 0) group_bound = expected = group_bound_of(plan, h, s);
             }
             switch (algo) {
-            case EG_ALGO_HASH: res = run_hash(plan, group_bound, expected, s); break;
+            case EG_ALGO_HASH: res = run_hash(plan, group_bound, expected, callers, s); break;
             case EG_ALGO_SORT: case EG_ALGO_SORT_OPT: res = run_sort(plan, h, false, s); break;
             case EG_ALGO_SORT_GFUR: res = run_sort(plan, h, true, s); break;
             case EG_ALGO_PARTITION: res = run_partition(plan, group_bound, expected, false, s); break;

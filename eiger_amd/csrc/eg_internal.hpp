@@ -232,8 +232,9 @@ struct HashTuning {
 };
 
 // expected: about how many groups there are, where more is known than the bound
-// (else the bound).
-Result run_hash(const Plan& plan, int64_t group_bound, int64_t expected, hipStream_t s, const HashTuning& t = HashTuning{});
+// (else the bound).  callers: the caller gave a bound below the rows.
+Result run_hash(const Plan& plan, int64_t group_bound, int64_t expected, bool callers, hipStream_t s,
+                const HashTuning& t = HashTuning{});
 
 // expected: as run_hash's.
 Result run_partition(const Plan& plan, int64_t group_bound, int64_t expected, bool gfur, hipStream_t s);

@@ -308,7 +308,7 @@ bool run_tiny(const Plan& plan, const HashTuning& t, hipStream_t s, Result& res)
 // the group count (at most 40 bytes a group for the benchmark's requests).
 constexpr int64_t kEarlyOutputRows = (int64_t)1 << 22;
 
-Result run_hash(const Plan& plan, int64_t group_bound, int64_t expected, hipStream_t s, const HashTuning& t)
+Result run_hash(const Plan& plan, int64_t group_bound, int64_t expected, bool callers, hipStream_t s, const HashTuning& t)
 {
     const int64_t n = plan.rows;
     const int nops = plan.spec.nops;
@@ -318,7 +318,12 @@ Result run_hash(const Plan& plan, int64_t group_bound, int64_t expected, hipStre
         Result res;
         if (KB == 4 ? run_tiny<4>(plan, t, s, res) : run_tiny<8>(plan, t, s, res)) return res;
     }
-    const HashLayout L = plan_hash_layout(nops, KB, group_bound, std::min(group_bound, expected), t);
+    // A caller's bound is the better guess of whether the keys outnumber the LDS
+    // slots: the estimate is short of skewed ones (2^28 rows, five states, 4096
+    // groups and bound at Zipf 1.2 2.57 -> 2.08 ms; uniform 7.43 -> 7.8).  A
+    // bound made of the estimate has its headroom on top (2^26 rows, 16 states,
+    // 1000 groups 1.06 ms by the estimate, 2.34 by the bound).
+    const HashLayout L = plan_hash_layout(nops, KB, group_bound, callers ? group_bound : std::min(group_bound, expected), t);
 
     bool vec = aligned16(plan.key.data);
     for (int c = 0; c < plan.spec.nvcols; ++c) vec = vec && aligned16(plan.spec.cols[c].data);
